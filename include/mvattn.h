@@ -555,6 +555,43 @@ int mv_paged_prefill_parts(const void* query, int64_t q_stride_tok, int64_t q_st
                            size_t workspace_bytes, void* stream);
 
 /*
+ * Query tokens an item of mv_paged_prefill_blocks may hold for this head
+ * shape and dtype (0: unsupported): as many as 128 query rows (tokens x query
+ * heads per kv head) hold, or 256 with `wide`, for the 16-bit types;
+ * mv_prefill_tokens_per_group for fp32.
+ */
+int mv_prefill_block_tokens(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                            int32_t dtype, int32_t wide);
+
+/* mv_paged_prefill_workspace_bytes for mv_paged_prefill_blocks (0 also for
+ * tokens_per_item outside 1 .. mv_prefill_block_tokens(.., wide)). */
+size_t mv_paged_prefill_blocks_workspace_bytes(int32_t num_units, int32_t max_parts,
+                                               int32_t tokens_per_item, int32_t num_q_heads,
+                                               int32_t num_kv_heads, int32_t head_dim,
+                                               int32_t dtype);
+
+/*
+ * mv_paged_prefill (max_parts 1: items of 4 ints, workspace unused) or
+ * mv_paged_prefill_parts (max_parts > 1: items of 8 ints) with items of up to
+ * tokens_per_item query tokens, 1 .. mv_prefill_block_tokens(.., wide). Items
+ * of more than mv_prefill_block_tokens(.., 0) tokens run with 256 query rows
+ * per work group: faster where the 128-row work groups would take more than
+ * one round over the CUs. Same math and contract otherwise.
+ */
+int mv_paged_prefill_blocks(const void* query, int64_t q_stride_tok, int64_t q_stride_head,
+                            const void* key, int64_t k_stride_tok, int64_t k_stride_head,
+                            const void* value, int64_t v_stride_tok, int64_t v_stride_head,
+                            const void* key_cache, const void* value_cache,
+                            const void* block_table, int32_t bt_is_i64, int64_t bt_stride,
+                            const int64_t* seqs, int32_t num_seqs, const int32_t* work_items,
+                            int32_t num_work_groups, int32_t tokens_per_item, int32_t num_units,
+                            int32_t max_parts, void* out, int64_t out_stride_tok,
+                            int64_t out_stride_head, float scale, int32_t num_q_heads,
+                            int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                            int64_t num_blocks, int32_t dtype, void* workspace,
+                            size_t workspace_bytes, void* stream);
+
+/*
  * Device-side plan of mv_paged_prefill for a launch of fixed size, e.g.
  * inside a captured graph where the step's lengths cannot be read back (no
  * counterpart in the reference: its prefill plans on the host). Inputs are

@@ -23,7 +23,7 @@ LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmvattn.so")
 
 SOURCES = ("mv_error.hip", "kv_cache_write.hip", "paged_decode.hip", "gather_paged_kv.hip",
-           "rope_kv_write.hip", "paged_prefill.hip")
+           "rope_kv_write.hip", "paged_prefill.hip", "paged_prefill_wide.hip")
 
 # gfx950 only. Packed-fp32 VALU ops are disabled: hipcc must not emit
 # v_pk_{add,mul,fma}_f32 (their results are not trusted on this hardware).

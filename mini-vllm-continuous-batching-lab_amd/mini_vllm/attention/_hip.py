@@ -175,6 +175,21 @@ SIGNATURES = {
         _F, _I32, _I32, _I32,      # scale, num_q_heads, num_kv_heads, head_dim
         _I32, _I64, _I32, _P,      # block_size, num_blocks, dtype, stream
     ]),
+    "mv_prefill_block_tokens": (ctypes.c_int, [_I32, _I32, _I32, _I32, _I32]),
+    "mv_paged_prefill_blocks_workspace_bytes": (ctypes.c_size_t, [_I32] * 7),
+    "mv_paged_prefill_blocks": (ctypes.c_int, [
+        _P, _I64, _I64,            # query, strides
+        _P, _I64, _I64,            # key, strides
+        _P, _I64, _I64,            # value, strides
+        _P, _P,                    # key_cache, value_cache
+        _P, _I32, _I64,            # block_table, bt_is_i64, bt_stride
+        _P, _I32, _P, _I32,        # seqs, num_seqs, work_items, num_work_groups
+        _I32, _I32, _I32,          # tokens_per_item, num_units, max_parts
+        _P, _I64, _I64,            # out, strides
+        _F, _I32, _I32, _I32,      # scale, num_q_heads, num_kv_heads, head_dim
+        _I32, _I64, _I32,          # block_size, num_blocks, dtype
+        _P, ctypes.c_size_t, _P,   # workspace, workspace_bytes, stream
+    ]),
     "mv_paged_prefill_workspace_bytes": (ctypes.c_size_t, [_I32, _I32, _I32, _I32, _I32, _I32]),
     "mv_paged_prefill_parts": (ctypes.c_int, [
         _P, _I64, _I64,            # query, strides

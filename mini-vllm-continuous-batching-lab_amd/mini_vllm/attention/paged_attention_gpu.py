@@ -1389,6 +1389,21 @@ def prefill_key_parts(key_ends: Sequence[int], cu_count: int,
     return out
 
 
+def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, units_of) -> int:
+    """Query tokens per work group of a prefill launch (``units_of(tokens)``
+    work groups, uncut): as many as 128 query rows hold while those work
+    groups fit the CUs in one round, else 256 (measured:
+    csrc/paged_prefill_wide.hip)."""
+    lib = _hip.load()
+    shape = (num_q_heads, num_kv_heads, head_dim, _hip.MV_DTYPE[dtype])
+    tokens = lib.mv_prefill_block_tokens(*shape, 0)
+    if tokens == 0:
+        raise RuntimeError(
+            f"prefill: {num_q_heads} query heads over {num_kv_heads} kv heads not supported"
+        )
+    return tokens if units_of(tokens) <= cu_count else lib.mv_prefill_block_tokens(*shape, 1)
+
+
 def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_q_heads,
                   num_kv_heads, head_dim, dtype, device):
     """Validated table and device work list of one step's prefill, built once:
@@ -1410,12 +1425,9 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
     hit = _cache_get("prefill", (block_table,), extra)
     if hit is not None:
         return hit
-    tpg = lib.mv_prefill_tokens_per_group(num_q_heads, num_kv_heads, head_dim,
-                                          _hip.MV_DTYPE[dtype])
-    if tpg == 0:
-        raise RuntimeError(
-            f"prefill: {num_q_heads} query heads over {num_kv_heads} kv heads not supported"
-        )
+    cus = _groups_per_cu(device, head_dim, dtype)[1]
+    tokens = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cus,
+                             lambda t: sum(-(-q // t) for q in qlens) * num_kv_heads)
     bt = block_table
     if bt.dim() != 2:
         bt = bt.reshape(-1, bt.shape[-1] if bt.dim() else 0)
@@ -1431,33 +1443,33 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
     start = 0
     for i, (r, c, ql) in enumerate(zip(rows, cached, qlens)):
         seqs.append((r, c, start, ql))
-        for t0 in range(0, ql, tpg):
-            nt = min(tpg, ql - t0)
+        for t0 in range(0, ql, tokens):
+            nt = min(tokens, ql - t0)
             for h in range(num_kv_heads):
                 items.append((i, h, t0, nt))
                 keys.append(c + t0 + nt)
         start += ql
     cap = int(os.environ.get("MVATTN_PREFILL_PARTS", PREFILL_MAX_PARTS))
-    parts = prefill_key_parts(keys, _groups_per_cu(device, head_dim, dtype)[1], cap)
-    max_parts = max((len(p) for p in parts), default=1)
-    split = None
+    parts = prefill_key_parts(keys, cus, cap)
+    units, max_parts = len(items), max((len(p) for p in parts), default=1)
     if max_parts > 1:
         groups = [(*items[u], k0, k1, u, p | len(pr) << 8 | max_parts << 16)
                   for u, pr in enumerate(parts) for p, (k0, k1) in enumerate(pr)]
         groups.sort(key=lambda g: g[4] - g[5])  # the most keys first
         work = torch.tensor(groups, dtype=torch.int32)
-        ws_bytes = lib.mv_paged_prefill_workspace_bytes(len(items), max_parts, num_q_heads,
-                                                        num_kv_heads, head_dim,
-                                                        _hip.MV_DTYPE[dtype])
-        # the plan's own merge workspace: its counters start at zero and every
-        # launch leaves them so; the layers of a step share it on one stream
-        split = (len(items), max_parts, torch.zeros(ws_bytes, dtype=torch.uint8, device=device))
     else:
         order = sorted(range(len(items)), key=lambda k: -keys[k])
         work = torch.tensor([items[k] for k in order] or [(0, 0, 0, 0)], dtype=torch.int32)
     meta = torch.tensor(seqs or [(0, 0, 0, 0)], dtype=torch.int64)
+    ws = None
+    if max_parts > 1:
+        ws_bytes = lib.mv_paged_prefill_blocks_workspace_bytes(
+            units, max_parts, tokens, num_q_heads, num_kv_heads, head_dim, _hip.MV_DTYPE[dtype])
+        # the plan's own merge workspace: its counters start at zero and every
+        # launch leaves them so; the layers of a step share it on one stream
+        ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device)
     plan = (bt, meta.to(device, non_blocking=True), work.to(device, non_blocking=True),
-            work.shape[0] if items else 0, split)
+            work.shape[0] if items else 0, tokens, units, max_parts, ws)
     _cache_put("prefill", (block_table,), extra, plan)
     return plan
 
@@ -1513,12 +1525,9 @@ def _prefill_device_plan(block_table, seq_indices, cached_len_before, query_len,
     hit = _cache_get("prefill_graph", tensors, extra)
     if hit is not None:
         return hit
-    tpg = lib.mv_prefill_tokens_per_group(num_q_heads, num_kv_heads, head_dim,
-                                          _hip.MV_DTYPE[dtype])
-    if tpg == 0:
-        raise RuntimeError(
-            f"prefill: {num_q_heads} query heads over {num_kv_heads} kv heads not supported"
-        )
+    tpg = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype,
+                          _groups_per_cu(device, head_dim, dtype)[1],
+                          lambda t: (-(-total_rows // t) + n) * num_kv_heads)
     bt = block_table
     if bt.dim() != 2:
         bt = bt.reshape(-1, bt.shape[-1] if bt.dim() else 0)
@@ -1556,7 +1565,7 @@ def _prefill_device_plan(block_table, seq_indices, cached_len_before, query_len,
             )
 
     _defer(capture, raise_prefill, status)
-    plan = (bt, seqs, work, cap)
+    plan = (bt, seqs, work, cap, tpg, 0, 1, None)
     _cache_put("prefill_graph", tensors, extra, plan)
     return plan
 
@@ -1614,10 +1623,9 @@ def hip_prefill_attention(
         out = torch.empty(total_q, num_q_heads, head_dim, dtype=query.dtype, device=device)
         if total_q == 0 or not rows:
             return out
-        bt, meta, work, n_work = _prefill_device_plan(
+        plan = _prefill_device_plan(
             block_table, rows, cached_len_before, query_len, total_q, block_size, num_blocks,
             num_q_heads, num_kv_heads, head_dim, query.dtype, device, capture)
-        split = None
     else:
         def host_ints(x):
             return x.tolist() if isinstance(x, torch.Tensor) else x
@@ -1632,25 +1640,26 @@ def hip_prefill_attention(
         out = torch.empty(total, num_q_heads, head_dim, dtype=query.dtype, device=device)
         if total == 0:
             return out
-        bt, meta, work, n_work, split = _prefill_plan(block_table, rows, cached, qlens,
-                                                      block_size, num_blocks, num_q_heads,
-                                                      num_kv_heads, head_dim, query.dtype, device)
+        plan = _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks,
+                             num_q_heads, num_kv_heads, head_dim, query.dtype, device)
 
     q = _aligned_rows(query)
     k = _aligned_rows(key)
     v = _aligned_rows(value)
-    head = (_ptr(q), q.stride(0), q.stride(1), _ptr(k), k.stride(0), k.stride(1),
+    bt, meta, work, n_work, tokens, units, max_parts, ws = plan
+    _hip.check(
+        lib.mv_paged_prefill_blocks(
+            _ptr(q), q.stride(0), q.stride(1), _ptr(k), k.stride(0), k.stride(1),
             _ptr(v), v.stride(0), v.stride(1), _ptr(key_cache), _ptr(value_cache),
             _ptr(bt) if bt.numel() else None, int(bt.dtype == torch.int64),
-            bt.stride(0) if bt.numel() else 0, _ptr(meta), len(rows), _ptr(work), n_work)
-    tail = (_ptr(out), out.stride(0), out.stride(1), float(head_dim ** -0.5), num_q_heads,
-            num_kv_heads, head_dim, block_size, num_blocks, _hip.MV_DTYPE[query.dtype])
-    if split is None:
-        _hip.check(lib.mv_paged_prefill(*head, *tail, _stream(device)), "mv_paged_prefill")
-    else:
-        units, max_parts, ws = split
-        _hip.check(lib.mv_paged_prefill_parts(*head, units, max_parts, *tail, _ptr(ws), ws.numel(),
-                                              _stream(device)), "mv_paged_prefill_parts")
+            bt.stride(0) if bt.numel() else 0, _ptr(meta), len(rows), _ptr(work), n_work,
+            tokens, units, max_parts, _ptr(out), out.stride(0), out.stride(1),
+            float(head_dim ** -0.5), num_q_heads, num_kv_heads, head_dim, block_size, num_blocks,
+            _hip.MV_DTYPE[query.dtype], _ptr(ws), ws.numel() if ws is not None else 0,
+            _stream(device),
+        ),
+        "mv_paged_prefill_blocks",
+    )
     return out
 
 

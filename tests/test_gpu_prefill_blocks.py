@@ -1,0 +1,103 @@
+"""mv_paged_prefill_blocks' two work-group sizes against the oracle.
+
+The 16-bit prefill runs 128 packed query rows per work group, or 256 where the
+128-row work groups would not fit the CUs in one round. Sizes here are the
+edges: chunks of one token, of a work group's tokens and one more or less;
+prefixes that end at, before and after a 16-key sub-tile, a 32-key tile and a
+stage (64 and 128 keys); wave rows that straddle the causal diagonal; query
+heads per kv head that do and do not divide the rows; output rows that are not
+16-byte aligned. Tolerance: the oracle tests' (16-bit rounding of outputs and
+probabilities).
+"""
+
+import pytest
+import torch
+
+from gpu_util import DEV, TOL, say
+from mini_vllm.attention import _hip
+from mini_vllm.attention import paged_attention_gpu as pag
+from test_gpu_prefill import _case, _ref, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _both_sizes(monkeypatch, c):
+    """The case's output with 128-row and with 256-row work groups."""
+    outs = []
+    for wide in (0, 1):
+        tokens = _hip.load().mv_prefill_block_tokens(c["hq"], c["hkv"], c["d"],
+                                                     _hip.MV_DTYPE[c["dtype"]], wide)
+        monkeypatch.setattr(pag, "_prefill_tokens", lambda *a, t=tokens: t)
+        outs.append(_run(c))
+    return outs
+
+
+@pytest.mark.parametrize("shape", [(14, 2, 64, 16, torch.bfloat16), (28, 4, 128, 16, torch.float16),
+                                   (8, 8, 64, 1, torch.float16), (16, 1, 128, 64, torch.bfloat16),
+                                   (9, 3, 128, 32, torch.bfloat16), (10, 5, 64, 8, torch.bfloat16)],
+                         ids=lambda s: f"{s[0]}-{s[1]}-{s[2]}-bs{s[3]}-{s[4]}")
+def test_edges_of_tiles_and_work_groups(monkeypatch, shape):
+    hq, hkv, d, bs, dt = shape
+    n_rep = hq // hkv
+    narrow, wide = 128 // n_rep, 256 // n_rep
+    cached = [0, 0, 15, 16, 31, 33, 63, 64, 127, 129, 255, 257, 0]
+    qlen = [1, narrow, narrow + 1, narrow - 1 or 1, wide, wide + 1, wide - 1 or 1, 2, 65, 1, 32, 33,
+            2 * wide + 3]
+    say("prefill block edges", shape, cached, qlen)
+    c = _case(hq, hkv, d, bs, dt, cached, qlen, seed=21, fused=True)
+    ref = _ref(c)
+    for out in _both_sizes(monkeypatch, c):
+        assert not torch.isnan(out).any()
+        err = (out - ref).abs().max().item()
+        assert err <= TOL[dt], err
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_wide_key_parts_and_sharp_scores(monkeypatch, d):
+    """Both sizes with their keys cut into parts (one long sequence), Q x 4:
+    tiles that leave the range of the softmax reference, merged across parts."""
+    say("prefill block parts", d)
+    c = _case(14, 2, d, 16, torch.bfloat16, [3000], [200], seed=22)
+    c["q"] = (c["q"] * 4).to(torch.bfloat16).float()
+    ref = _ref(c)
+    for out in _both_sizes(monkeypatch, c):
+        err = (out - ref).abs().max().item()
+        assert err <= TOL[torch.bfloat16], err
+
+
+@pytest.mark.parametrize("wide", [0, 1])
+def test_output_rows_not_16_byte_aligned(wide):
+    """The C ABI takes any output strides: element stores give the same bits
+    as the 16-byte stores."""
+    hq, hkv, d, bs, t = 14, 2, 64, 16, 70
+    say("prefill blocks unaligned output", wide)
+    lib = _hip.load()
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(t, h, d, generator=g).to(torch.bfloat16).to(DEV) for h in (hq, hkv, hkv))
+    kc = torch.zeros(4, hkv, bs, d, dtype=torch.bfloat16, device=DEV)
+    tokens = lib.mv_prefill_block_tokens(hq, hkv, d, 2, wide)
+    work = torch.tensor([(0, h, t0, min(tokens, t - t0)) for t0 in range(0, t, tokens)
+                         for h in range(hkv)], dtype=torch.int32, device=DEV)
+    seqs = torch.tensor([[0, 0, 0, t]], dtype=torch.int64, device=DEV)
+    bt = torch.zeros(1, 1, dtype=torch.int64, device=DEV)
+    outs = []
+    for pad in (0, 1):
+        out = torch.empty(t, hq, d + pad, dtype=torch.bfloat16, device=DEV)
+        rc = lib.mv_paged_prefill_blocks(
+            q.data_ptr(), *q.stride()[:2], k.data_ptr(), *k.stride()[:2], v.data_ptr(),
+            *v.stride()[:2], kc.data_ptr(), kc.data_ptr(), bt.data_ptr(), 1, 1, seqs.data_ptr(), 1,
+            work.data_ptr(), work.shape[0], tokens, work.shape[0], 1, out.data_ptr(),
+            *out.stride()[:2], d ** -0.5, hq, hkv, d, bs, 4, 2, None, 0,
+            torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        outs.append(out[..., :d].clone())
+    assert torch.equal(outs[0], outs[1])
+
+
+def test_size_rule(monkeypatch):
+    """256 rows exactly where the 128-row work groups exceed the CUs."""
+    args = (14, 2, 64, torch.bfloat16, 256)
+    assert pag._prefill_tokens(*args, lambda t: 256) == 18
+    assert pag._prefill_tokens(*args, lambda t: 257) == 36
+    assert pag._prefill_tokens(14, 2, 64, torch.float32, 256, lambda t: 10 ** 6) == 16
