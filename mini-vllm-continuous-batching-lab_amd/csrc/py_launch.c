@@ -2,7 +2,7 @@
  * _mvlaunch: CPython fast-call wrappers of the C-ABI entry points that the
  * Python wrappers call once per layer or step (mv_paged_decode_write,
  * mv_paged_decode, mv_kv_cache_write, mv_rope_kv_cache_write,
- * mv_decode_plan; include/mvattn.h).
+ * mv_decode_plan, mv_paged_prefill_blocks; include/mvattn.h).
  *
  * ctypes converts every argument through libffi: about 5 us for the 35
  * arguments of mv_paged_decode_write on the build host, a third of an eager
@@ -37,12 +37,14 @@ typedef __typeof__(&mv_paged_decode) decode_fn;
 typedef __typeof__(&mv_kv_cache_write) cache_write_fn;
 typedef __typeof__(&mv_rope_kv_cache_write) rope_write_fn;
 typedef __typeof__(&mv_decode_plan) plan_fn;
+typedef __typeof__(&mv_paged_prefill_blocks) prefill_fn;
 
 static decode_write_fn g_decode_write;
 static rope_write_fn g_rope_write;
 static plan_fn g_plan;
 static decode_fn g_decode;
 static cache_write_fn g_cache_write;
+static prefill_fn g_prefill;
 
 /* A pointer argument: an int address, or None for a null pointer. */
 static void* arg_ptr(PyObject* o) { return o == Py_None ? NULL : PyLong_AsVoidPtr(o); }
@@ -279,6 +281,56 @@ static PyObject* plan(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   return PyLong_FromLong(rc);
 }
 
+/* Arguments of mv_paged_prefill_blocks, in its order. */
+static PyObject* prefill(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  (void)self;
+  if (check_nargs("prefill", n, 34, (const void*)g_prefill)) return NULL;
+  const void* query = arg_ptr(a[0]);
+  const int64_t q_st = arg_i64(a[1]), q_sh = arg_i64(a[2]);
+  const void* key = arg_ptr(a[3]);
+  const int64_t k_st = arg_i64(a[4]), k_sh = arg_i64(a[5]);
+  const void* value = arg_ptr(a[6]);
+  const int64_t v_st = arg_i64(a[7]), v_sh = arg_i64(a[8]);
+  const void* key_cache = arg_ptr(a[9]);
+  const void* value_cache = arg_ptr(a[10]);
+  const void* block_table = arg_ptr(a[11]);
+  const int32_t bt_i64 = arg_i32(a[12]);
+  const int64_t bt_stride = arg_i64(a[13]);
+  const int64_t* seqs = (const int64_t*)arg_ptr(a[14]);
+  const int32_t num_seqs = arg_i32(a[15]);
+  const int32_t* work = (const int32_t*)arg_ptr(a[16]);
+  const int32_t groups = arg_i32(a[17]), tokens = arg_i32(a[18]), units = arg_i32(a[19]);
+  const int32_t max_parts = arg_i32(a[20]);
+  void* out = arg_ptr(a[21]);
+  const int64_t o_st = arg_i64(a[22]), o_sh = arg_i64(a[23]);
+  const float scale = arg_f32(a[24]);
+  const int32_t hq = arg_i32(a[25]), hkv = arg_i32(a[26]), d = arg_i32(a[27]), bs = arg_i32(a[28]);
+  const int64_t num_blocks = arg_i64(a[29]);
+  const int32_t dtype = arg_i32(a[30]);
+  void* ws = arg_ptr(a[31]);
+  const size_t ws_bytes = arg_size(a[32]);
+  void* stream = arg_ptr(a[33]);
+  if (PyErr_Occurred()) return NULL;
+  const int rc = g_prefill(query, q_st, q_sh, key, k_st, k_sh, value, v_st, v_sh, key_cache,
+                           value_cache, block_table, bt_i64, bt_stride, seqs, num_seqs, work, groups,
+                           tokens, units, max_parts, out, o_st, o_sh, scale, hq, hkv, d, bs,
+                           num_blocks, dtype, ws, ws_bytes, stream);
+  return PyLong_FromLong(rc);
+}
+
+/* bind_prefill(prefill): the address of mv_paged_prefill_blocks. */
+static PyObject* bind_prefill(PyObject* self, PyObject* address) {
+  (void)self;
+  void* p = PyLong_AsVoidPtr(address);
+  if (PyErr_Occurred()) return NULL;
+  if (!p) {
+    PyErr_SetString(PyExc_ValueError, "_mvlaunch.bind_prefill: null address");
+    return NULL;
+  }
+  g_prefill = (prefill_fn)p;
+  Py_RETURN_NONE;
+}
+
 /* bind(decode_write, decode, cache_write, rope_write, plan): the entry
  * points' addresses in the loaded libmvattn.so (ctypes resolves them). */
 static PyObject* bind(PyObject* self, PyObject* const* a, Py_ssize_t n) {
@@ -318,6 +370,9 @@ static PyMethodDef methods[] = {
      "mv_rope_kv_cache_write with its 31 arguments"},
     {"plan", (PyCFunction)(void (*)(void))plan, METH_FASTCALL,
      "mv_decode_plan with its 20 arguments"},
+    {"prefill", (PyCFunction)(void (*)(void))prefill, METH_FASTCALL,
+     "mv_paged_prefill_blocks with its 34 arguments"},
+    {"bind_prefill", (PyCFunction)bind_prefill, METH_O, "bind mv_paged_prefill_blocks"},
     {NULL, NULL, 0, NULL},
 };
 

@@ -223,6 +223,7 @@ decode = None        # mv_paged_decode
 cache_write = None   # mv_kv_cache_write
 rope_write = None    # mv_rope_kv_cache_write
 plan = None          # mv_decode_plan
+prefill = None       # mv_paged_prefill_blocks
 # mv_paged_decode_write from a step's packed words (step_words()) and one
 # layer's tensors; None without _mvlaunch (the wrappers then call
 # decode_write with all 35 arguments).
@@ -248,9 +249,10 @@ def step_words(slots: int, rope_cos: int, rope_sin: int, work: int, ids: int, id
 
 
 def _bind_calls(lib: ctypes.CDLL) -> None:
-    global decode_write, decode, cache_write, rope_write, plan, decode_write_step
+    global decode_write, decode, cache_write, rope_write, plan, prefill, decode_write_step
     ctypes_calls = (lib.mv_paged_decode_write, lib.mv_paged_decode, lib.mv_kv_cache_write,
                     lib.mv_rope_kv_cache_write, lib.mv_decode_plan)
+    prefill = lib.mv_paged_prefill_blocks
     try:
         from . import _mvlaunch
     except ImportError:
@@ -269,6 +271,9 @@ def _bind_calls(lib: ctypes.CDLL) -> None:
     decode_write, decode, cache_write, rope_write, plan = (
         _mvlaunch.decode_write, _mvlaunch.decode, _mvlaunch.cache_write, _mvlaunch.rope_write,
         _mvlaunch.plan)
+    if hasattr(_mvlaunch, "prefill"):
+        _mvlaunch.bind_prefill(ctypes.cast(prefill, ctypes.c_void_p).value)
+        prefill = _mvlaunch.prefill
     decode_write_step = (_mvlaunch.decode_write_step
                          if getattr(_mvlaunch, "STEP_WORDS", None) == STEP_WORDS else None)
 

@@ -30,6 +30,7 @@ import weakref
 from dataclasses import dataclass, field
 from typing import Any, List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from . import _hip
@@ -1138,15 +1139,6 @@ def _check_positions(positions: torch.Tensor, max_positions: int) -> None:
     _cache_put(name, (positions,), extra, True)
 
 
-def _rope_operand(x: torch.Tensor) -> torch.Tensor:
-    """x with 16-byte aligned, head_dim-contiguous rows (a copy only if not)."""
-    eb = x.element_size()
-    if (x.stride(2) != 1 or (x.stride(0) * eb) % 16 or (x.stride(1) * eb) % 16
-            or x.data_ptr() % 16):
-        x = x.contiguous()
-    return x
-
-
 def hip_rope_kv_cache_write(
     query: Optional[torch.Tensor],
     key: torch.Tensor,
@@ -1237,34 +1229,38 @@ def hip_rope_kv_cache_write(
         if not capture:
             _cache_put("rope_step", given, step_extra, (slot_mapping, positions))
 
-    q_out = None
+    # (views and aligned copies are bound to names: they live until the launch)
+    q_out = k_out = None
+    qp = qo = ko = vp = 0
+    q_st = q_sh = qo_st = qo_sh = ko_st = ko_sh = v_st = v_sh = 0
     if query is not None:
-        query = _rope_operand(query)
+        query, qp, q_st, q_sh = _row_args(query)
         q_out = query if inplace else torch.empty_like(query, memory_format=torch.contiguous_format)
-    k_out = torch.empty_like(key, memory_format=torch.contiguous_format) if return_key else None
+        qo = q_out.data_ptr()
+        qo_st, qo_sh, _ = q_out.stride()
+    if return_key:
+        k_out = torch.empty_like(key, memory_format=torch.contiguous_format)
+        ko = k_out.data_ptr()
+        ko_st, ko_sh, _ = k_out.stride()
     if num_tokens == 0:
         return q_out, k_out
-    key = _rope_operand(key)
+    key, kp, k_st, k_sh = _row_args(key)
     if write:
-        value = _rope_operand(value)
-    if cos.stride(1) != 1 or sin.stride(1) != 1 or cos.stride(0) != sin.stride(0):
+        value, vp, v_st, v_sh = _row_args(value)
+    cos_st, sin_st = cos.stride(), sin.stride()
+    if cos_st[1] != 1 or sin_st[1] != 1 or cos_st[0] != sin_st[0]:
         cos, sin = cos.contiguous(), sin.contiguous()
+        cos_st = cos.stride()
     _hip.load()  # binds _hip.rope_write
     _hip.check(
         _hip.rope_write(
-            _ptr(query), query.stride(0) if query is not None else 0,
-            query.stride(1) if query is not None else 0,
-            _ptr(q_out), q_out.stride(0) if q_out is not None else 0,
-            q_out.stride(1) if q_out is not None else 0,
-            _ptr(key), key.stride(0), key.stride(1),
-            _ptr(k_out), k_out.stride(0) if k_out is not None else 0,
-            k_out.stride(1) if k_out is not None else 0,
-            _ptr(value) if write else None, value.stride(0) if write else 0,
-            value.stride(1) if write else 0,
-            _ptr(key_cache), _ptr(value_cache), _ptr(slot_mapping) if write else None,
-            _ptr(positions), _ptr(cos), _ptr(sin), cos.stride(0), cos.shape[0],
-            num_tokens, num_q_heads, num_kv_heads, head_dim, block_size if write else 0,
-            num_blocks, _hip.MV_DTYPE[dtype], _stream(device),
+            qp or None, q_st, q_sh, qo or None, qo_st, qo_sh, kp, k_st, k_sh, ko or None, ko_st,
+            ko_sh, vp or None, v_st, v_sh, key_cache.data_ptr() if write else None,
+            value_cache.data_ptr() if write else None,
+            slot_mapping.data_ptr() if write else None, positions.data_ptr(), cos.data_ptr(),
+            sin.data_ptr(), cos_st[0], cos.shape[0], num_tokens, num_q_heads, num_kv_heads,
+            head_dim, block_size if write else 0, num_blocks, _hip.MV_DTYPE[dtype],
+            _stream(device),
         ),
         "mv_rope_kv_cache_write",
     )
@@ -1389,6 +1385,55 @@ def prefill_key_parts(key_ends: Sequence[int], cu_count: int,
     return out
 
 
+def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int, tpg: int,
+                 cu_count: int, max_parts: int):
+    """Sequence records and work list of a prefill launch.
+
+    Units are (sequence, kv head, block of ``tpg`` chunk tokens). Returns
+    ``(seqs, work, units, parts)``: int64 [n, 4] (0, cached, first chunk row,
+    chunk tokens), int32 [slots, 4 or 8] (8 when some unit is cut into parts,
+    ``prefill_key_parts``), the number of units and the most parts of one.
+    """
+    cached = np.asarray(cached, dtype=np.int64).reshape(-1)
+    qlens = np.asarray(qlens, dtype=np.int64).reshape(-1)
+    n = len(qlens)
+    seqs = np.zeros((max(n, 1), 4), dtype=np.int64)
+    if n:
+        seqs[:, 1], seqs[:, 3] = cached, qlens
+        seqs[1:, 2] = np.cumsum(qlens)[:-1]
+    blocks = np.maximum(-(-qlens // tpg), 0)
+    nu = int(blocks.sum()) * num_kv_heads
+    if nu == 0:
+        return seqs, np.zeros((0, 4), dtype=np.int32), 0, 1
+    # (sequence, token block) from each sequence's last block (the most
+    # keys), every kv head of it in a row
+    seq = np.repeat(np.arange(n), blocks)
+    t0 = (np.repeat(np.cumsum(blocks), blocks) - 1 - np.arange(len(seq))) * tpg
+    nt = np.minimum(tpg, qlens[seq] - t0)
+    unit_keys = cached[seq] + t0 + nt
+    items = np.empty((len(seq), num_kv_heads, 4), dtype=np.int32)
+    items[:, :, 0], items[:, :, 2], items[:, :, 3] = seq[:, None], t0[:, None], nt[:, None]
+    items[:, :, 1] = np.arange(num_kv_heads)
+    items = items.reshape(nu, 4)
+    keys = np.repeat(unit_keys, num_kv_heads)
+    most = 1
+    if nu < cu_count:  # the parts of prefill_key_parts, unit by unit
+        kb = -(-keys // PREFILL_PART_KEYS)
+        count = np.clip(kb // 2, 1, max(1, min(max_parts, cu_count // nu)))
+        most = int(count.max())
+    if most > 1:
+        unit = np.repeat(np.arange(nu), count)
+        part = np.arange(len(unit)) - np.repeat(np.cumsum(count) - count, count)
+        kb, cnt = kb[unit], count[unit]
+        first = part * kb // cnt * PREFILL_PART_KEYS
+        end = np.where(part + 1 == cnt, keys[unit], (part + 1) * kb // cnt * PREFILL_PART_KEYS)
+        split = np.stack([first, end, unit, part | cnt << 8 | most << 16], axis=1)
+        items = np.concatenate([items[unit], split.astype(np.int32)], axis=1)
+        keys = end - first
+    work = items[np.argsort(-keys, kind="stable")]  # the most keys first
+    return seqs, work, nu, most
+
+
 def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, units_of) -> int:
     """Query tokens per work group of a prefill launch (``units_of(tokens)``
     work groups, uncut): as many as 128 query rows hold while those work
@@ -1427,7 +1472,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         return hit
     cus = _groups_per_cu(device, head_dim, dtype)[1]
     tokens = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cus,
-                             lambda t: sum(-(-q // t) for q in qlens) * num_kv_heads)
+                             lambda t: sum(-(-q // t) for q in qlens if q > 0) * num_kv_heads)
     bt = block_table
     if bt.dim() != 2:
         bt = bt.reshape(-1, bt.shape[-1] if bt.dim() else 0)
@@ -1439,28 +1484,10 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         bt = bt.to(torch.int64)
     if bt.numel() and bt.stride(1) != 1:
         bt = bt.contiguous()
-    seqs, items, keys = [], [], []
-    start = 0
-    for i, (r, c, ql) in enumerate(zip(rows, cached, qlens)):
-        seqs.append((r, c, start, ql))
-        for t0 in range(0, ql, tokens):
-            nt = min(tokens, ql - t0)
-            for h in range(num_kv_heads):
-                items.append((i, h, t0, nt))
-                keys.append(c + t0 + nt)
-        start += ql
-    cap = int(os.environ.get("MVATTN_PREFILL_PARTS", PREFILL_MAX_PARTS))
-    parts = prefill_key_parts(keys, cus, cap)
-    units, max_parts = len(items), max((len(p) for p in parts), default=1)
-    if max_parts > 1:
-        groups = [(*items[u], k0, k1, u, p | len(pr) << 8 | max_parts << 16)
-                  for u, pr in enumerate(parts) for p, (k0, k1) in enumerate(pr)]
-        groups.sort(key=lambda g: g[4] - g[5])  # the most keys first
-        work = torch.tensor(groups, dtype=torch.int32)
-    else:
-        order = sorted(range(len(items)), key=lambda k: -keys[k])
-        work = torch.tensor([items[k] for k in order] or [(0, 0, 0, 0)], dtype=torch.int32)
-    meta = torch.tensor(seqs or [(0, 0, 0, 0)], dtype=torch.int64)
+    seqs, work, units, max_parts = prefill_work(
+        cached, qlens, num_kv_heads, tokens, cus,
+        int(os.environ.get("MVATTN_PREFILL_PARTS", PREFILL_MAX_PARTS)))
+    seqs[:, 0] = rows
     ws = None
     if max_parts > 1:
         ws_bytes = lib.mv_paged_prefill_blocks_workspace_bytes(
@@ -1468,8 +1495,9 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         # the plan's own merge workspace: its counters start at zero and every
         # launch leaves them so; the layers of a step share it on one stream
         ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device)
-    plan = (bt, meta.to(device, non_blocking=True), work.to(device, non_blocking=True),
-            work.shape[0] if items else 0, tokens, units, max_parts, ws)
+    plan = (bt, torch.from_numpy(seqs).to(device, non_blocking=True),
+            torch.from_numpy(work).to(device, non_blocking=True), len(work), tokens, units,
+            max_parts, ws)
     _cache_put("prefill", (block_table,), extra, plan)
     return plan
 
@@ -1503,6 +1531,18 @@ def _device_i64(x, n: int, device: torch.device) -> torch.Tensor:
     for i, v in enumerate(vals):
         t[i].fill_(v)
     return t
+
+
+def _host_lengths(cached_len_before, query_len) -> Tuple[List[int], List[int]]:
+    """Both length lists as Python ints; two device tensors are read back in
+    one copy (each read waits for the layers enqueued before it)."""
+    c, q = cached_len_before, query_len
+    if (isinstance(c, torch.Tensor) and isinstance(q, torch.Tensor) and c.is_cuda
+            and c.device == q.device and c.dtype == q.dtype and c.shape == q.shape and c.dim() == 1):
+        c, q = torch.stack((c, q)).tolist()
+    else:
+        c, q = (x.tolist() if isinstance(x, torch.Tensor) else x for x in (c, q))
+    return [int(x) for x in c], [int(x) for x in q]
 
 
 def _prefill_device_plan(block_table, seq_indices, cached_len_before, query_len, total_rows,
@@ -1615,7 +1655,7 @@ def hip_prefill_attention(
     assert key_cache.is_contiguous() and value_cache.is_contiguous()
     assert query.device.type == "cuda"
     device = query.device
-    lib = _hip.load()
+    _hip.load()  # binds _hip.prefill
     capture = _capture_id(device)
     rows = [int(r) for r in seq_indices]
     if capture:
@@ -1627,11 +1667,7 @@ def hip_prefill_attention(
             block_table, rows, cached_len_before, query_len, total_q, block_size, num_blocks,
             num_q_heads, num_kv_heads, head_dim, query.dtype, device, capture)
     else:
-        def host_ints(x):
-            return x.tolist() if isinstance(x, torch.Tensor) else x
-
-        cached = [int(c) for c in host_ints(cached_len_before)]
-        qlens = [int(q) for q in host_ints(query_len)]
+        cached, qlens = _host_lengths(cached_len_before, query_len)
         assert len(rows) == len(cached) == len(qlens)
         total = sum(qlens)
         assert total <= total_q and total <= key.shape[0], (
@@ -1643,17 +1679,19 @@ def hip_prefill_attention(
         plan = _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks,
                              num_q_heads, num_kv_heads, head_dim, query.dtype, device)
 
-    q = _aligned_rows(query)
-    k = _aligned_rows(key)
-    v = _aligned_rows(value)
+    # (the views are bound to names: an aligned copy lives until the launch)
+    q, qp, q_st, q_sh = _row_args(query)
+    k, kp, k_st, k_sh = _row_args(key)
+    v, vp, v_st, v_sh = _row_args(value)
     bt, meta, work, n_work, tokens, units, max_parts, ws = plan
+    has_bt = bt.numel() > 0
+    o_st, o_sh, _ = out.stride()
     _hip.check(
-        lib.mv_paged_prefill_blocks(
-            _ptr(q), q.stride(0), q.stride(1), _ptr(k), k.stride(0), k.stride(1),
-            _ptr(v), v.stride(0), v.stride(1), _ptr(key_cache), _ptr(value_cache),
-            _ptr(bt) if bt.numel() else None, int(bt.dtype == torch.int64),
-            bt.stride(0) if bt.numel() else 0, _ptr(meta), len(rows), _ptr(work), n_work,
-            tokens, units, max_parts, _ptr(out), out.stride(0), out.stride(1),
+        _hip.prefill(
+            qp, q_st, q_sh, kp, k_st, k_sh, vp, v_st, v_sh, key_cache.data_ptr(),
+            value_cache.data_ptr(), bt.data_ptr() if has_bt else None,
+            int(bt.dtype == torch.int64), bt.stride(0) if has_bt else 0, meta.data_ptr(), len(rows),
+            work.data_ptr(), n_work, tokens, units, max_parts, out.data_ptr(), o_st, o_sh,
             float(head_dim ** -0.5), num_q_heads, num_kv_heads, head_dim, block_size, num_blocks,
             _hip.MV_DTYPE[query.dtype], _ptr(ws), ws.numel() if ws is not None else 0,
             _stream(device),

@@ -44,3 +44,68 @@ def test_wide_partials_are_published_before_the_counter(tmp_path):
     assert len(ks) == 8, sorted(ks)  # 2 dtypes x 2 head dims x 2 table types
     for name, ins in ks.items():
         check_handoff(name, ins)
+
+
+def test_launcher_passes_every_argument_in_order():
+    """The fast-call wrapper against a stand-in for mv_paged_prefill_blocks."""
+    import ctypes
+
+    from mini_vllm.attention import _mvlaunch
+
+    restype, argtypes = _hip.SIGNATURES["mv_paged_prefill_blocks"]
+    got = []
+    stand_in = ctypes.CFUNCTYPE(restype, *argtypes)(lambda *a: got.append(a) or 5)
+    args = [1000 + i for i in range(len(argtypes))]
+    args[argtypes.index(ctypes.c_float)] = 0.125
+    real = ctypes.cast(_hip.load().mv_paged_prefill_blocks, ctypes.c_void_p).value
+    try:
+        _mvlaunch.bind_prefill(ctypes.cast(stand_in, ctypes.c_void_p).value)
+        assert _mvlaunch.prefill(*args) == 5
+        assert list(got[0]) == args
+        with pytest.raises(TypeError, match="34 arguments"):
+            _mvlaunch.prefill(*args[:-1])
+    finally:
+        _mvlaunch.bind_prefill(real)
+
+
+def _work_by_loops(cached, qlens, hkv, tokens, cus, max_parts):
+    """The work list's definition, unit by unit."""
+    from mini_vllm.attention.paged_attention_gpu import prefill_key_parts
+
+    items, keys = [], []
+    for i, (c, q) in enumerate(zip(cached, qlens)):
+        for t0 in range(0, q, tokens):
+            for h in range(hkv):
+                items.append((i, h, t0, min(tokens, q - t0)))
+                keys.append(c + t0 + items[-1][3])
+    return items, prefill_key_parts(keys, cus, max_parts)
+
+
+@pytest.mark.parametrize("cached,qlens,hkv,tokens", [
+    ([1536] * 4, [512] * 4, 2, 18), ([0], [37], 2, 18), ([3584], [512], 2, 18), ([0], [8192], 4, 36),
+    ([5, 0, 700], [0, 3, 41], 8, 16), ([0, 2000, 17], [900, 1, 33], 1, 128), ([7], [0], 2, 18),
+])
+def test_work_list_holds_every_unit_and_part_once(cached, qlens, hkv, tokens):
+    from mini_vllm.attention.paged_attention_gpu import prefill_work
+
+    seqs, work, units, most = prefill_work(cached, qlens, hkv, tokens, 256, 8)
+    items, parts = _work_by_loops(cached, qlens, hkv, tokens, 256, 8)
+    starts = [sum(qlens[:i]) for i in range(len(qlens))]
+    assert seqs.tolist() == [[0, c, s, q] for c, s, q in zip(cached, starts, qlens)]
+    assert units == len(items)
+    assert most == max((len(p) for p in parts), default=1)
+    rows = work.tolist()
+    if most == 1:
+        assert sorted(map(tuple, rows)) == sorted(items)
+        size = [cached[r[0]] + r[2] + r[3] for r in rows]
+    else:
+        got = {}
+        for r in rows:
+            assert r[7] >> 16 == most and (r[7] >> 8) & 0xff == len(parts[items.index(tuple(r[:4]))])
+            got.setdefault((tuple(r[:4]), r[6]), {})[r[7] & 0xff] = (r[4], r[5])
+        assert len({u for _, u in got}) == len(got) == units and {u for _, u in got} == set(range(units))
+        for (item, _), ranges in got.items():
+            want = parts[items.index(item)]
+            assert [ranges[p] for p in range(len(want))] == want
+        size = [r[5] - r[4] for r in rows]
+    assert size == sorted(size, reverse=True)  # the most keys first
