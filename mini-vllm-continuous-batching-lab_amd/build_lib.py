@@ -116,6 +116,39 @@ def build_launcher(verbose: bool = False) -> str:
     return out
 
 
+TORCH_CALLS_SOURCE = os.path.join(CSRC, "py_torch.cpp")
+
+
+def build_torch_calls(verbose: bool = False) -> str:
+    """Compile the native per-layer launches (``csrc/py_torch.cpp``, host C++
+    on torch's headers) into ``mini_vllm/attention/_mvtorch<EXT_SUFFIX>``;
+    returns its path. Without it the Python wrappers do the same work."""
+    import sysconfig
+
+    import torch
+
+    out = os.path.join(LAUNCHER_DIR, "_mvtorch" + sysconfig.get_config_var("EXT_SUFFIX"))
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no C++ compiler (g++) for the per-layer launches")
+    root = os.path.dirname(torch.__file__)
+    fd, tmp = tempfile.mkstemp(prefix="_mvtorch.", suffix=".so.tmp", dir=LAUNCHER_DIR)
+    os.close(fd)
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(root, "include"), "-I", sysconfig.get_paths()["include"],
+           "-I", INCLUDE, TORCH_CALLS_SOURCE, "-o", tmp, "-L", os.path.join(root, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        os.unlink(tmp)
+        raise RuntimeError(f"per-layer launches build failed ({proc.returncode}):\n{proc.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 if __name__ == "__main__":
     import argparse
 
@@ -128,3 +161,4 @@ if __name__ == "__main__":
         ap.error("a variant needs --out: lib/libmvattn.so is the default build")
     print(build(verbose=True, defines=args.define, out=args.out))
     print(build_launcher(verbose=True))
+    print(build_torch_calls(verbose=True))

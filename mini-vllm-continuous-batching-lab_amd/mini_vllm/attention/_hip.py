@@ -229,6 +229,14 @@ prefill = None       # mv_paged_prefill_blocks
 # decode_write with all 35 arguments).
 decode_write_step = None
 
+# _mvtorch (csrc/py_torch.cpp), bound to the loaded library: a layer's checks,
+# output allocation and launch in one native call. None where it is not built.
+# It stands in for the launcher's functions: the wrappers use it while the
+# entry points above are those of `launcher` (_mvlaunch), so that a function put
+# in their place gets the calls.
+native = None
+launcher = None
+
 # The step words' layout (csrc/py_launch.c): mv_paged_decode_write's
 # step-constant arguments in its order, one little-endian 64-bit word each,
 # the scale as a double.
@@ -246,6 +254,38 @@ def step_words(slots: int, rope_cos: int, rope_sin: int, work: int, ids: int, id
                        ids or 0, ids_cap, groups, part_tokens, max_parts, counters or 0, scale,
                        num_seqs, hq, hkv, head_dim, block_size, num_blocks, dtype_code, ws or 0,
                        ws_bytes)
+
+
+# The words of _mvtorch.decode and _mvtorch.prefill: the step-constant
+# arguments of mv_paged_decode and mv_paged_prefill_blocks in their order, then
+# for prefill the device index.
+DECODE_WORDS_FORMAT = "<7qd9q"
+PREFILL_WORDS_FORMAT = "<10qd9q"
+
+
+def decode_words(*args) -> bytes:
+    return struct.pack(DECODE_WORDS_FORMAT, *(a or 0 for a in args))
+
+
+def prefill_words(*args) -> bytes:
+    return struct.pack(PREFILL_WORDS_FORMAT, *(a or 0 for a in args))
+
+
+def _bind_native(lib: ctypes.CDLL, mvlaunch) -> None:
+    global native, launcher
+    launcher = mvlaunch
+    try:
+        from . import _mvtorch
+    except ImportError:
+        native = None
+        return
+    if _mvtorch.ABI != ABI_VERSION:
+        native = None
+        return
+    _mvtorch.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
+        lib.mv_paged_decode_write, lib.mv_paged_decode, lib.mv_kv_cache_write,
+        lib.mv_rope_kv_cache_write, lib.mv_paged_prefill_blocks)))
+    native = _mvtorch
 
 
 def _bind_calls(lib: ctypes.CDLL) -> None:
@@ -274,6 +314,7 @@ def _bind_calls(lib: ctypes.CDLL) -> None:
     if hasattr(_mvlaunch, "prefill"):
         _mvlaunch.bind_prefill(ctypes.cast(prefill, ctypes.c_void_p).value)
         prefill = _mvlaunch.prefill
+    _bind_native(lib, _mvlaunch)
     decode_write_step = (_mvlaunch.decode_write_step
                          if getattr(_mvlaunch, "STEP_WORDS", None) == STEP_WORDS else None)
 

@@ -77,6 +77,11 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(index).cuda_stream
 
 
+# (without the Python wrapper around it, ~0.3 us a call)
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing",
+                     torch.cuda.is_current_stream_capturing)
+
+
 def _is_pow2(v: int) -> bool:
     return v > 0 and (v & (v - 1)) == 0
 
@@ -172,7 +177,7 @@ def _check_workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor
 def _capture_id(device: torch.device) -> int:
     """Id of the graph capture the current stream of ``device`` is in (HIP's
     capture id, nonzero), or 0 when it is not being captured."""
-    if not torch.cuda.is_current_stream_capturing():
+    if not _capturing():
         return 0
     cid = ctypes.c_uint64(0)
     _hip.check(_hip.load().mv_stream_capture_id(_stream(device), ctypes.byref(cid)),
@@ -324,6 +329,20 @@ def hip_cache_write(
     sliced out of a fused QKV output) as long as ``head_dim`` is
     contiguous; no staging copy is made.
     """
+    # The other layers of an eager step: checked and launched in native code
+    # (None: not the plain case, all of it below).
+    entry = getattr(_state, "write_step", None)
+    native = _hip.native
+    if entry is not None and native is not None and _hip.cache_write is _hip.launcher.cache_write:
+        seen, slots = entry
+        if native.seen(seen.refs, seen.versions, slot_mapping) and not _capturing():
+            total_slots, device = seen.extra
+            done = native.cache_write(slots, total_slots, key, value, key_cache, value_cache,
+                                      slot_mapping, block_size, _stream(device))
+            if done is not None:
+                if done is not True:
+                    _hip.check(done, "mv_kv_cache_write")
+                return
     num_tokens, num_kv_heads, head_dim = key.shape
     assert key.shape == value.shape, f"key {key.shape} != value {value.shape}"
     assert key_cache.shape == value_cache.shape
@@ -394,6 +413,9 @@ class DecodePlan:
     partition_tokens: int
     # merge workspace bytes per query-head count (asked of the library once)
     ws_bytes: dict = field(default_factory=dict)
+    # (packed launch words, the workspace they point at) per query-head
+    # count, for the other layers of an eager step
+    words: dict = field(default_factory=dict)
 
 
 # The plan aims for as many work groups as the device holds at once (work
@@ -868,6 +890,54 @@ def _fused_step_prepare(block_table: torch.Tensor, kv_len_after: torch.Tensor, b
     return plan, slots, fused_ok, rows
 
 
+def _decode_native(query, key_cache, value_cache, block_table, kv_len_after, block_size, new_key,
+                   new_value, slot_mapping, positions, cos, sin) -> Optional[torch.Tensor]:
+    """A layer of an eager step whose plan and checks are made (the same,
+    unmodified metadata tensors): its own checks and its launch in native
+    code. None where the step is not known, the call is not the plain case or
+    a graph is being captured: the wrapper's own path runs it."""
+    native = _hip.native
+    if query.dim() != 3:
+        return None
+    if new_key is None:
+        entry = getattr(_state, "plan", None)
+        if _hip.decode is not _hip.launcher.decode:
+            return None
+        if entry is None or not native.seen(entry[0].refs, entry[0].versions, block_table,
+                                            kv_len_after):
+            return None
+        words = entry[1].words.get(query.shape[1])
+    else:
+        entry = getattr(_state, "fused_step", None)
+        if _hip.decode_write_step is not _hip.launcher.decode_write_step:
+            return None
+        if entry is None or not native.seen(entry[0].refs, entry[0].versions, slot_mapping,
+                                            block_table, kv_len_after):
+            return None
+        rows = 0
+        if positions is not None:
+            rope = getattr(_state, "rope_rows", None)
+            if rope is None or not native.seen(rope[0].refs, rope[0].versions, positions, cos, sin):
+                return None
+            rows = id(rope[1][0])
+        words = entry[1][2].get((query.shape[1], rows))
+    if words is None or _capturing():
+        return None
+    packed, ws, device = words[0], words[1], entry[0].extra[2]
+    if ws is not None and _WORKSPACES.get(device) is not ws:
+        return None
+    if new_key is None:
+        output = native.decode(packed, query, key_cache, value_cache, block_table, kv_len_after,
+                               block_size, device.index, _stream(device))
+    else:
+        output = native.decode_write(packed, query, key_cache, value_cache, block_table,
+                                     kv_len_after, block_size, new_key, new_value, positions,
+                                     device.index, _stream(device))
+    if type(output) is int:
+        _hip.check(output, "mv_paged_decode" if new_key is None else "mv_paged_decode_write")
+    return output
+
+
 def hip_decode_attention(
     query: torch.Tensor,
     key_cache: torch.Tensor,
@@ -919,6 +989,11 @@ def hip_decode_attention(
     output and pool bit-identical to ``hip_rope_kv_cache_write`` followed by
     this call on the rotated query.
     """
+    if _hip.native is not None:  # the other layers of an eager step
+        output = _decode_native(query, key_cache, value_cache, block_table, kv_len_after,
+                                block_size, new_key, new_value, slot_mapping, positions, cos, sin)
+        if output is not None:
+            return output
     # (The per-call checks read each attribute once: this wrapper runs once
     # per layer, and its host time exceeds the kernel's when it does not.)
     total_decode, num_q_heads, head_dim = query.shape
@@ -1050,6 +1125,15 @@ def hip_decode_attention(
             "mv_paged_decode_write",
         )
         return output
+    if not capture and _hip.native is not None:
+        # the other layers of the step launch from these words
+        plan.words[num_q_heads] = (
+            _hip.decode_words(
+                _ptr(plan.work), _ptr(plan.block_ids), plan.block_ids.numel(), plan.num_groups,
+                plan.partition_tokens, plan.max_parts, _ptr(plan.counters),
+                float(head_dim ** -0.5), total_decode, num_q_heads, num_kv_heads, head_dim,
+                block_size, num_blocks, _hip.MV_DTYPE[dtype], _ptr(ws),
+                ws.numel() if ws is not None else 0), ws)
     _hip.check(
         _hip.decode(
             _ptr(query), query.stride(0), query.stride(1),
@@ -1173,6 +1257,22 @@ def hip_rope_kv_cache_write(
     reference: ``AssertionError`` (shapes, dtypes, duplicate slots),
     ``IndexError`` (slot or position out of range).
     """
+    # The other layers of an eager step: checked and launched in native code
+    # (None: not the plain case, all of it below).
+    entry = getattr(_state, "rope_step", None)
+    native = _hip.native
+    if (entry is not None and native is not None and key_cache is not None and not inplace
+            and _hip.rope_write is _hip.launcher.rope_write):
+        seen, (slots, checked) = entry
+        if native.seen(seen.refs, seen.versions, slot_mapping, positions) and not _capturing():
+            total_slots, rows, device = seen.extra
+            done = native.rope_write(slots, checked, total_slots, rows, query, key, value, positions,
+                                     cos, sin, key_cache, value_cache, slot_mapping, block_size,
+                                     return_key, _stream(device))
+            if done is not None:
+                if type(done) is int:
+                    _hip.check(done, "mv_rope_kv_cache_write")
+                return done
     num_tokens, num_kv_heads, head_dim = key.shape
     dtype, device = key.dtype, key.device
     assert device.type == "cuda", f"key.device must be cuda, got {device}"
@@ -1498,6 +1598,12 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
     plan = (bt, torch.from_numpy(seqs).to(device, non_blocking=True),
             torch.from_numpy(work).to(device, non_blocking=True), len(work), tokens, units,
             max_parts, ws)
+    has_bt = bt.numel() > 0
+    plan += (_hip.prefill_words(
+        _ptr(bt) if has_bt else None, int(bt.dtype == torch.int64), bt.stride(0) if has_bt else 0,
+        _ptr(plan[1]), len(rows), _ptr(plan[2]), len(work), tokens, units, max_parts,
+        float(head_dim ** -0.5), num_q_heads, num_kv_heads, head_dim, block_size, num_blocks,
+        _hip.MV_DTYPE[dtype], _ptr(ws), ws.numel() if ws is not None else 0, device.index),)
     _cache_put("prefill", (block_table,), extra, plan)
     return plan
 
@@ -1605,7 +1711,7 @@ def _prefill_device_plan(block_table, seq_indices, cached_len_before, query_len,
             )
 
     _defer(capture, raise_prefill, status)
-    plan = (bt, seqs, work, cap, tpg, 0, 1, None)
+    plan = (bt, seqs, work, cap, tpg, 0, 1, None, None)
     _cache_put("prefill_graph", tensors, extra, plan)
     return plan
 
@@ -1673,17 +1779,24 @@ def hip_prefill_attention(
         assert total <= total_q and total <= key.shape[0], (
             f"{total} chunk tokens, query has {total_q} rows, key {key.shape[0]}"
         )
-        out = torch.empty(total, num_q_heads, head_dim, dtype=query.dtype, device=device)
         if total == 0:
-            return out
+            return torch.empty(total, num_q_heads, head_dim, dtype=query.dtype, device=device)
         plan = _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks,
                              num_q_heads, num_kv_heads, head_dim, query.dtype, device)
+        if _hip.native is not None and _hip.prefill is _hip.launcher.prefill:
+            out = _hip.native.prefill(plan[8], query, key, value, key_cache, value_cache, total,
+                                      _stream(device))
+            if out is not None:
+                if type(out) is int:
+                    _hip.check(out, "mv_paged_prefill_blocks")
+                return out
+        out = torch.empty(total, num_q_heads, head_dim, dtype=query.dtype, device=device)
 
     # (the views are bound to names: an aligned copy lives until the launch)
     q, qp, q_st, q_sh = _row_args(query)
     k, kp, k_st, k_sh = _row_args(key)
     v, vp, v_st, v_sh = _row_args(value)
-    bt, meta, work, n_work, tokens, units, max_parts, ws = plan
+    bt, meta, work, n_work, tokens, units, max_parts, ws, _ = plan
     has_bt = bt.numel() > 0
     o_st, o_sh, _ = out.stride()
     _hip.check(
