@@ -57,6 +57,7 @@ extern "C" {
 /* Status words written by mv_kv_slots_check (int32[2], device memory). */
 #define MV_SLOTS_OUT_OF_RANGE 0 /* # slots < -1 or >= num_blocks*block_size */
 #define MV_SLOTS_DUPLICATES 1   /* # (i < j) pairs with slot[i] == slot[j] >= 0 */
+#define MV_SLOTS_POSITIONS 2 /* mv_kv_slots_positions_check only */
 
 /* Status words written by mv_decode_write_check (int32[2], device memory). */
 #define MV_WRITE_CHECK_OWN_SLOT 0 /* # slots not at their own sequence's kv_len - 1 */
@@ -144,6 +145,17 @@ int mv_kv_cache_write(const void* key, int64_t key_stride_tok, int64_t key_strid
 size_t mv_kv_slots_check_workspace_bytes(int64_t num_tokens);
 int mv_kv_slots_check(const int64_t* slot_mapping, int64_t num_tokens, int64_t total_slots,
                       int32_t* status, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * mv_kv_slots_check and mv_positions_check over the same tokens in one launch
+ * (two above 4096 tokens) and one status: status[0], [1] as mv_kv_slots_check,
+ * status[2] = positions outside [0, max_positions). positions: int64
+ * [num_tokens], not null. Same workspace and limits as mv_kv_slots_check.
+ */
+int mv_kv_slots_positions_check(const int64_t* slot_mapping, int64_t num_tokens,
+                                int64_t total_slots, const int64_t* positions,
+                                int64_t max_positions, int32_t* status, void* workspace,
+                                size_t workspace_bytes, void* stream);
 
 /*
  * Precondition check of mv_paged_decode_write (the fused decode + KV write;

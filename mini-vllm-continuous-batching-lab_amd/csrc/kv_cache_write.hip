@@ -105,49 +105,61 @@ constexpr int kSlotsGridThreads = 256;
 constexpr int64_t kSlotsMax = (int64_t(1) << (64 - kSlotCountShift)) - 1;  // count field
 
 __global__ __launch_bounds__(kSlotsCheckThreads) void slots_check_lds_kernel(
-    const int64_t* slots, int32_t n, int64_t total_slots, uint32_t hmask, int32_t* status) {
+    const int64_t* slots, int32_t n, int64_t total_slots, const int64_t* positions, int64_t max_positions,
+    uint32_t hmask, int32_t* status) {
   __shared__ uint64_t table[kSlotsLdsEntries];
-  __shared__ int s_bad;
+  __shared__ int s_bad, s_bad_pos;
   __shared__ unsigned long long s_pairs;
   for (uint32_t i = threadIdx.x; i <= hmask; i += kSlotsCheckThreads) table[i] = 0;
-  if (threadIdx.x == 0) { s_bad = 0; s_pairs = 0; }
+  if (threadIdx.x == 0) { s_bad = 0; s_bad_pos = 0; s_pairs = 0; }
   __syncthreads();
-  int bad = 0;
+  int bad = 0, bad_pos = 0;
   uint64_t pairs = 0;
   for (int x = threadIdx.x; x < n; x += kSlotsCheckThreads) {
     const int64_t s = slots[x];
+    if (positions) {
+      const int64_t p = positions[x];
+      bad_pos += p < 0 || p >= max_positions;
+    }
     if (s == -1) continue;
     if (s < 0 || s >= total_slots) { ++bad; continue; }
     pairs += count_insert(table, hmask, static_cast<uint64_t>(s) + 1);
   }
   if (bad) atomicAdd(&s_bad, bad);
+  if (bad_pos) atomicAdd(&s_bad_pos, bad_pos);
   if (pairs) atomicAdd(&s_pairs, static_cast<unsigned long long>(pairs));
   __syncthreads();
   if (threadIdx.x == 0) {
     status[MV_SLOTS_OUT_OF_RANGE] = s_bad;
     status[MV_SLOTS_DUPLICATES] = saturate_i32(s_pairs);
+    if (positions) status[MV_SLOTS_POSITIONS] = s_bad_pos;
   }
 }
 
 __global__ __launch_bounds__(kSlotsGridThreads) void slots_clear_kernel(uint64_t* table,
                                                                         int64_t entries,
-                                                                        int32_t* status) {
+                                                                        int32_t* status,
+                                                                        int32_t words) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kSlotsGridThreads;
   for (int64_t i = blockIdx.x * int64_t(kSlotsGridThreads) + threadIdx.x; i < entries; i += stride)
     table[i] = 0;
-  if (blockIdx.x == 0 && threadIdx.x < 2) status[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < words) status[threadIdx.x] = 0;
 }
 
 __global__ __launch_bounds__(kSlotsGridThreads) void slots_check_grid_kernel(
-    const int64_t* slots, int64_t n, int64_t total_slots, uint64_t* table, uint32_t hmask,
-    int32_t* status) {
-  __shared__ int s_bad;
+    const int64_t* slots, int64_t n, int64_t total_slots, const int64_t* positions, int64_t max_positions,
+    uint64_t* table, uint32_t hmask, int32_t* status) {
+  __shared__ int s_bad, s_bad_pos;
   __shared__ unsigned long long s_pairs;
-  if (threadIdx.x == 0) { s_bad = 0; s_pairs = 0; }
+  if (threadIdx.x == 0) { s_bad = 0; s_bad_pos = 0; s_pairs = 0; }
   __syncthreads();
   const int64_t x = blockIdx.x * int64_t(kSlotsGridThreads) + threadIdx.x;
   if (x < n) {
     const int64_t s = slots[x];
+    if (positions) {
+      const int64_t p = positions[x];
+      if (p < 0 || p >= max_positions) atomicAdd(&s_bad_pos, 1);
+    }
     if (s != -1) {
       if (s < 0 || s >= total_slots) {
         atomicAdd(&s_bad, 1);
@@ -160,6 +172,7 @@ __global__ __launch_bounds__(kSlotsGridThreads) void slots_check_grid_kernel(
   __syncthreads();
   if (threadIdx.x == 0) {
     if (s_bad) atomicAdd(&status[MV_SLOTS_OUT_OF_RANGE], s_bad);
+    if (s_bad_pos) atomicAdd(&status[MV_SLOTS_POSITIONS], s_bad_pos);
     if (s_pairs) {  // saturating add
       int32_t* p = &status[MV_SLOTS_DUPLICATES];
       int32_t old = *p;
@@ -322,10 +335,14 @@ extern "C" size_t mv_kv_slots_check_workspace_bytes(int64_t num_tokens) {
   return static_cast<size_t>(pow2_at_least(2 * num_tokens)) * sizeof(uint64_t);
 }
 
-extern "C" int mv_kv_slots_check(const int64_t* slot_mapping, int64_t num_tokens,
-                                 int64_t total_slots, int32_t* status, void* workspace,
-                                 size_t workspace_bytes, void* stream) {
-  using namespace mv;
+namespace mv {
+namespace {
+
+// The slot check, with the positions check in the same launch where positions
+// is not null.
+int slots_check(const int64_t* slot_mapping, int64_t num_tokens, int64_t total_slots,
+                const int64_t* positions, int64_t max_positions, int32_t* status, void* workspace,
+                size_t workspace_bytes, void* stream) {
   if (!status) return fail(MV_ERR_INVALID_ARGUMENT, "mv_kv_slots_check: null status");
   if (num_tokens < 0 || total_slots < 0)
     return fail(MV_ERR_INVALID_ARGUMENT, "mv_kv_slots_check: negative size");
@@ -341,7 +358,7 @@ extern "C" int mv_kv_slots_check(const int64_t* slot_mapping, int64_t num_tokens
   if (num_tokens <= kSlotsLdsMax) {
     const uint32_t entries = pow2_at_least(std::max<int64_t>(64, 2 * num_tokens));
     slots_check_lds_kernel<<<1, kSlotsCheckThreads, 0, s>>>(
-        slot_mapping, static_cast<int32_t>(num_tokens), total_slots, entries - 1, status);
+        slot_mapping, static_cast<int32_t>(num_tokens), total_slots, positions, max_positions, entries - 1, status);
     return check_launch("mv_kv_slots_check");
   }
   const size_t need = mv_kv_slots_check_workspace_bytes(num_tokens);
@@ -354,12 +371,32 @@ extern "C" int mv_kv_slots_check(const int64_t* slot_mapping, int64_t num_tokens
   uint64_t* table = static_cast<uint64_t*>(workspace);
   const int64_t entries = static_cast<int64_t>(need / sizeof(uint64_t));
   const int64_t clear_groups = std::min<int64_t>((entries + kSlotsGridThreads - 1) / kSlotsGridThreads, 1024);
-  slots_clear_kernel<<<static_cast<unsigned>(clear_groups), kSlotsGridThreads, 0, s>>>(table, entries,
-                                                                                     status);
+  slots_clear_kernel<<<static_cast<unsigned>(clear_groups), kSlotsGridThreads, 0, s>>>(table, entries, status,
+                                                                                     positions ? 3 : 2);
   const int64_t groups = (num_tokens + kSlotsGridThreads - 1) / kSlotsGridThreads;
   slots_check_grid_kernel<<<static_cast<unsigned>(groups), kSlotsGridThreads, 0, s>>>(
-      slot_mapping, num_tokens, total_slots, table, static_cast<uint32_t>(entries - 1), status);
+      slot_mapping, num_tokens, total_slots, positions, max_positions, table, static_cast<uint32_t>(entries - 1), status);
   return check_launch("mv_kv_slots_check");
+}
+
+}  // namespace
+}  // namespace mv
+
+extern "C" int mv_kv_slots_check(const int64_t* slot_mapping, int64_t num_tokens,
+                                 int64_t total_slots, int32_t* status, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+  return mv::slots_check(slot_mapping, num_tokens, total_slots, nullptr, 0, status, workspace,
+                         workspace_bytes, stream);
+}
+
+extern "C" int mv_kv_slots_positions_check(const int64_t* slot_mapping, int64_t num_tokens,
+                                           int64_t total_slots, const int64_t* positions,
+                                           int64_t max_positions, int32_t* status, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+  if (!positions)
+    return mv::fail(MV_ERR_INVALID_ARGUMENT, "mv_kv_slots_positions_check: null positions");
+  return mv::slots_check(slot_mapping, num_tokens, total_slots, positions, max_positions, status,
+                         workspace, workspace_bytes, stream);
 }
 
 extern "C" size_t mv_decode_write_check_workspace_bytes(int32_t num_seqs) {

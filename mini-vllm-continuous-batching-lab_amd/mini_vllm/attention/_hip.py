@@ -73,6 +73,7 @@ SIGNATURES = {
     ]),
     "mv_kv_slots_check_workspace_bytes": (_SZ, [_I64]),
     "mv_kv_slots_check": (ctypes.c_int, [_P, _I64, _I64, _P, _P, _SZ, _P]),
+    "mv_kv_slots_positions_check": (ctypes.c_int, [_P, _I64, _I64, _P, _I64, _P, _P, _SZ, _P]),
     "mv_decode_write_check_workspace_bytes": (_SZ, [_I32]),
     "mv_decode_write_check": (ctypes.c_int, [
         _P, _P, _I32, _I64,        # slot_mapping, block_table, bt_is_i64, bt_stride

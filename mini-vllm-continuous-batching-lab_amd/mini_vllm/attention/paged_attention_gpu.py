@@ -259,6 +259,67 @@ def invalidate_cached_metadata() -> None:
 # ============================================================================
 
 
+def _slots_error(total_slots: int):
+    """Raises for a slot check's status words (out of range, duplicate pairs)."""
+
+    def raise_slots(st) -> None:
+        bad, dups = st[:2]
+        if bad:
+            raise IndexError(
+                f"slot_mapping has {bad} slot(s) out of range [0, {total_slots}) "
+                f"(-1 marks a skipped token)"
+            )
+        if dups:
+            raise AssertionError(
+                f"Duplicate slots in slot_mapping: {dups} duplicate pair(s). "
+                f"The HIP cache write forbids duplicate slots."
+            )
+
+    return raise_slots
+
+
+def _check_slots_positions(slots: torch.Tensor, total_slots: int, positions: torch.Tensor,
+                           max_positions: int, capture: int) -> None:
+    """``_check_slots`` and ``_check_positions`` of a step's new tokens (both
+    int64, contiguous, on the device): one launch and one read-back where
+    neither is known, same errors in the same order, same caches."""
+    g = "_graph" if capture else ""
+    slots_extra, pos_extra = (total_slots, capture), (max_positions, capture)
+    n = slots.numel()
+    if (n == 0 or _cache_get("slots" + g, (slots,), slots_extra) is not None
+            or _cache_get("positions" + g, (positions,), pos_extra) is not None):
+        _check_slots(slots, total_slots, capture=capture)
+        _check_positions(positions, max_positions)
+        return
+    lib = _hip.load()
+    status = torch.empty(3, dtype=torch.int32, device=slots.device)
+    ws_bytes = lib.mv_kv_slots_check_workspace_bytes(n)
+    ws = _check_workspace(slots.device, ws_bytes)
+    _hip.check(
+        lib.mv_kv_slots_positions_check(
+            _ptr(slots), n, total_slots, _ptr(positions), max_positions, _ptr(status), _ptr(ws),
+            ws_bytes, _stream(slots.device),
+        ),
+        "mv_kv_slots_positions_check",
+    )
+    raise_slots = _slots_error(total_slots)
+
+    def raise_positions(st) -> None:
+        if st[2]:
+            raise IndexError(f"{st[2]} position(s) outside the rotary tables [0, {max_positions})")
+
+    if capture:
+        _defer(capture, raise_slots, status)
+        _defer(capture, raise_positions, status)
+    else:
+        st = status.tolist()
+        raise_slots(st)
+    _cache_put("slots" + g, (slots,), slots_extra, True)
+    if not capture:
+        raise_positions(st)
+    _cache_put("positions" + g, (positions,), pos_extra, True)
+
+
 def _check_slots(slot_mapping: torch.Tensor, total_slots: int,
                  capture: Optional[int] = None) -> None:
     """Raise like the reference for out-of-range or duplicate slots.
@@ -289,19 +350,7 @@ def _check_slots(slot_mapping: torch.Tensor, total_slots: int,
         "mv_kv_slots_check",
     )
 
-    def raise_slots(st) -> None:
-        bad, dups = st
-        if bad:
-            raise IndexError(
-                f"slot_mapping has {bad} slot(s) out of range [0, {total_slots}) "
-                f"(-1 marks a skipped token)"
-            )
-        if dups:
-            raise AssertionError(
-                f"Duplicate slots in slot_mapping: {dups} duplicate pair(s). "
-                f"The HIP cache write forbids duplicate slots."
-            )
-
+    raise_slots = _slots_error(total_slots)
     if capture:
         _defer(capture, raise_slots, status)
     else:
@@ -1319,13 +1368,16 @@ def hip_rope_kv_cache_write(
             if slot_mapping.dtype != torch.int64:
                 slot_mapping = slot_mapping.to(torch.int64)
             slot_mapping = slot_mapping.contiguous()
-            _check_slots(slot_mapping, num_blocks * block_size, capture=capture)
         if positions.device != device:
             positions = positions.to(device)
         if positions.dtype != torch.int64:
             positions = positions.to(torch.int64)
         positions = positions.contiguous()
-        _check_positions(positions, cos.shape[0])
+        if write:
+            _check_slots_positions(slot_mapping, num_blocks * block_size, positions, cos.shape[0],
+                                   capture)
+        else:
+            _check_positions(positions, cos.shape[0])
         if not capture:
             _cache_put("rope_step", given, step_extra, (slot_mapping, positions))
 

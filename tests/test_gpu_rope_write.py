@@ -247,3 +247,44 @@ def test_backend_sub_layer_method():
     torch.cuda.synchronize()
     for x, y in ((ref, out), (kc, pool.key_caches[0]), (vc, pool.value_caches[0])):
         assert torch.equal(bits(x.cpu()), bits(y.cpu()))
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 4096, 4097, 9000])
+def test_slots_and_positions_checked_together(n):
+    """One launch and status for both checks, below and above the LDS table's
+    4096 tokens: the counts of the separate checks, and the errors in the
+    slots-first order."""
+    from mini_vllm.attention import _hip
+    from mini_vllm.attention import paged_attention_gpu as pg
+
+    say("slots and positions check", n)
+    lib = _hip.load()
+    g = torch.Generator().manual_seed(n)
+    total, max_pos = 20000, 500
+    for bad_slots, dups, bad_pos in ((0, 0, 0), (0, 0, 1), (1, 0, 1), (0, 1, 1)):
+        slots = torch.randperm(total, generator=g)[:n]
+        pos = torch.randint(0, max_pos, (n,), generator=g)
+        if bad_slots:
+            slots[n // 2] = total
+        if dups and n > 1:
+            slots[-1] = slots[0]
+        if bad_pos:
+            pos[0], pos[-1] = -1, max_pos
+        slots, pos = slots.to(DEV), pos.to(DEV)
+        status = torch.full((4,), 77, dtype=torch.int32, device=DEV)
+        nbytes = lib.mv_kv_slots_check_workspace_bytes(n)
+        ws = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=DEV)
+        rc = lib.mv_kv_slots_positions_check(slots.data_ptr(), n, total, pos.data_ptr(), max_pos,
+                                             status.data_ptr(), ws.data_ptr(), nbytes,
+                                             torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        want = [bad_slots, 1 if dups and n > 1 else 0,
+                (2 if n > 1 else 1) if bad_pos else 0, 77]
+        assert status.tolist() == want
+        pg.invalidate_cached_metadata()
+        error = IndexError if want[0] else AssertionError if want[1] else IndexError
+        if any(want[:3]):
+            with pytest.raises(error, match="slot" if want[0] or want[1] else "position"):
+                pg._check_slots_positions(slots, total, pos, max_pos, 0)
+        else:
+            pg._check_slots_positions(slots, total, pos, max_pos, 0)
