@@ -604,6 +604,18 @@ int mv_paged_prefill_blocks(const void* query, int64_t q_stride_tok, int64_t q_s
                             size_t workspace_bytes, void* stream);
 
 /*
+ * The table check of a prefill plan: status[i] (int32[num_seqs], device) = 1
+ * where sequence i of seqs (see mv_paged_prefill) has a table row outside
+ * [0, bt_rows), a cached prefix that is negative or longer than max_blocks
+ * blocks, or an entry among the prefix's blocks that is not a pool block (the
+ * reference's "insufficient", cache_read.py:60-67), else 0.
+ */
+int mv_prefill_prefix_check(const int64_t* seqs, int32_t num_seqs, const void* block_table,
+                            int32_t bt_is_i64, int64_t bt_stride, int32_t bt_rows,
+                            int32_t max_blocks, int32_t block_size, int64_t num_blocks,
+                            int32_t* status, void* stream);
+
+/*
  * Device-side plan of mv_paged_prefill for a launch of fixed size, e.g.
  * inside a captured graph where the step's lengths cannot be read back (no
  * counterpart in the reference: its prefill plans on the host). Inputs are

@@ -176,6 +176,11 @@ SIGNATURES = {
         _F, _I32, _I32, _I32,      # scale, num_q_heads, num_kv_heads, head_dim
         _I32, _I64, _I32, _P,      # block_size, num_blocks, dtype, stream
     ]),
+    "mv_prefill_prefix_check": (ctypes.c_int, [
+        _P, _I32, _P, _I32, _I64,  # seqs, num_seqs, block_table, bt_is_i64, bt_stride
+        _I32, _I32, _I32, _I64,    # bt_rows, max_blocks, block_size, num_blocks
+        _P, _P,                    # status, stream
+    ]),
     "mv_prefill_block_tokens": (ctypes.c_int, [_I32, _I32, _I32, _I32, _I32]),
     "mv_paged_prefill_blocks_workspace_bytes": (ctypes.c_size_t, [_I32] * 7),
     "mv_paged_prefill_blocks": (ctypes.c_int, [

@@ -1605,7 +1605,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
                   num_kv_heads, head_dim, dtype, device):
     """Validated table and device work list of one step's prefill, built once:
     the layers of a step pass the same (unmodified) block table and lengths,
-    so only the first call validates (one host copy of the table) and
+    so only the first call validates (on the device, one read-back) and
     uploads; the others reuse it.
 
     Work groups are (sequence, kv head, first token, tokens), the most keys
@@ -1628,9 +1628,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
     bt = block_table
     if bt.dim() != 2:
         bt = bt.reshape(-1, bt.shape[-1] if bt.dim() else 0)
-    if any(cached):
-        _check_prefix_tables(bt.detach().to("cpu", torch.int64), rows, cached, block_size,
-                             num_blocks)
+    host_bt = bt  # (on its own device, as given)
     bt = bt.to(device)
     if bt.dtype not in (torch.int32, torch.int64):
         bt = bt.to(torch.int64)
@@ -1640,6 +1638,23 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         cached, qlens, num_kv_heads, tokens, cus,
         int(os.environ.get("MVATTN_PREFILL_PARTS", PREFILL_MAX_PARTS)))
     seqs[:, 0] = rows
+    meta = torch.from_numpy(seqs).to(device, non_blocking=True)
+    if any(cached):
+        # every entry the prefixes need is a pool block: checked on the device,
+        # what is wrong looked up on the host
+        status = torch.empty(len(rows), dtype=torch.int32, device=device)
+        _hip.check(
+            lib.mv_prefill_prefix_check(
+                _ptr(meta), len(rows), _ptr(bt) if bt.numel() else None,
+                int(bt.dtype == torch.int64), bt.stride(0) if bt.numel() else 0,
+                bt.shape[0] if bt.numel() else 0, bt.shape[1] if bt.numel() else 0, block_size,
+                num_blocks, _ptr(status), _stream(device),
+            ),
+            "mv_prefill_prefix_check",
+        )
+        if any(status.tolist()):
+            _check_prefix_tables(host_bt.detach().to("cpu", torch.int64), rows, cached, block_size,
+                                 num_blocks)
     ws = None
     if max_parts > 1:
         ws_bytes = lib.mv_paged_prefill_blocks_workspace_bytes(
@@ -1647,7 +1662,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         # the plan's own merge workspace: its counters start at zero and every
         # launch leaves them so; the layers of a step share it on one stream
         ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device)
-    plan = (bt, torch.from_numpy(seqs).to(device, non_blocking=True),
+    plan = (bt, meta,
             torch.from_numpy(work).to(device, non_blocking=True), len(work), tokens, units,
             max_parts, ws)
     has_bt = bt.numel() > 0

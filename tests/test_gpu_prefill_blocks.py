@@ -101,3 +101,41 @@ def test_size_rule(monkeypatch):
     assert pag._prefill_tokens(*args, lambda t: 256) == 18
     assert pag._prefill_tokens(*args, lambda t: 257) == 36
     assert pag._prefill_tokens(14, 2, 64, torch.float32, 256, lambda t: 10 ** 6) == 16
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32], ids=str)
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_prefix_entries_are_checked_on_the_device(dtype, where):
+    """The plan's table check against its definition on the host: rows and
+    prefixes outside the table, entries at the pool's edges, entries past the
+    prefix that do not count; tables of either type, on either side."""
+    say("prefill prefix check", dtype, where)
+    hq, hkv, d, bs, nb = 14, 2, 64, 16, 40
+    good = torch.arange(2 * 6).view(2, 6)
+    cases = [(good, [0, 1], [96, 5], True), (good, [1, 0], [0, 81], True),
+             (good, [0, 2], [16, 0], False), (good, [0, -1], [16, 0], False),
+             (good, [0, 1], [97, 0], False)]
+    for at, ok in ((4, False), (5, True)):  # block 4 holds token 79, block 5 is past 80 tokens
+        for entry in (-1, nb):
+            t = good.clone()
+            t[1, at] = entry
+            cases.append((t, [0, 1], [16, 80], ok))
+    t = torch.full((2, 600), nb - 1)  # more entries than threads
+    t[0, 599] = nb
+    cases += [(t, [1, 0], [9600, 9584], True), (t, [1, 0], [9600, 9585], False)]
+    q = torch.zeros(2, hq, d, dtype=torch.bfloat16, device=DEV)
+    k = torch.zeros(2, hkv, d, dtype=torch.bfloat16, device=DEV)
+    kc = torch.zeros(nb, hkv, bs, d, dtype=torch.bfloat16, device=DEV)
+    for table, rows, cached, ok in cases:
+        table = table.to(dtype)
+        table = table.to(DEV) if where == "device" else table
+        try:
+            pag._check_prefix_tables(table.cpu().long(), rows, cached, bs, nb)
+            assert ok
+        except IndexError:
+            assert not ok
+        if ok:
+            pag.hip_prefill_attention(q, k, k, kc, kc, table, rows, cached, [1, 1], bs)
+        else:
+            with pytest.raises(IndexError, match="insufficient"):
+                pag.hip_prefill_attention(q, k, k, kc, kc, table, rows, cached, [1, 1], bs)
