@@ -990,15 +990,35 @@ struct PieceRules {
   int64_t target;
   int l_cap, l_min, l_top, l_fair;
 };
+// Few units (fewer than half the CUs): every piece beyond the first costs its
+// unit's merge 0.14-0.2 us (the last group to finish loads every partial), and
+// a wave 0.4 us (fp32: 0.85) per tile of its own piece, so the shortest pieces
+// that fill the slots are not the fastest. The bound is at least the root of
+// half the longest sequence's tiles, near where the two costs meet (half:
+// fp32's side of it), to the nearest whole round of the four waves: 5 tiles
+// take two rounds (fp32, 1 sequence of 1024: 6.6 us at 4 tiles, 7.6 at 5). Up
+// to kFewTilesPerCU tiles per CU one group per CU is enough: merges, not
+// streaming, are the bound there. us per call, before -> after (14 / 2 heads x
+// 64 bf16 unless noted): 4 sequences of 4096 15.1 -> 9.1, 8 of 2048 12.7 ->
+// 9.0, 2 of 8192 19.8 -> 9.5, 16 of 4096 (32 tiles per CU) 12.5 -> 10.6; 28 / 4
+// heads x 128, 2 of 4096 19.2 -> 11.3; fp32, 8 of 2048 14.3 -> 10.7; up to 1024
+// tokens the bound stays 4. Above 32 tiles per CU two groups per CU stream as
+// fast (16 of 8192: 16.5 either way), and from half the CUs' units on a unit
+// has few pieces anyway (32 of 2048, 28 / 4 x 128: 24.6 us either way).
+constexpr int kFewTilesPerCU = 32;
 __device__ inline PieceRules piece_rules(int groups_per_cu, int cu_count, int bs_log2, int64_t units,
                                          int64_t total_tiles, int most_tiles, int hkv) {
   PieceRules r;
-  const int per_cu = units <= cu_count ? vmin(kFewUnitsPerCU, vmax(1, groups_per_cu))
+  const bool few = 2 * units < cu_count;
+  const int few_per_cu = few && total_tiles * hkv <= static_cast<int64_t>(kFewTilesPerCU) * cu_count ? 1 : kFewUnitsPerCU;
+  const int per_cu = units <= cu_count ? vmin(few_per_cu, vmax(1, groups_per_cu))
                                        : vmin(kManyUnitsPerCU, vmax(1, groups_per_cu));
   r.target = static_cast<int64_t>(per_cu) * vmax(1, cu_count);
   r.l_cap = static_cast<int>(vmax<int64_t>(
       1, vmin<int64_t>(INT_MAX / 32, ((static_cast<int64_t>(kIdCap - 1)) << bs_log2) / kTile)));
   r.l_min = vmin(r.l_cap, vmax(kWaves, (most_tiles + kMaxParts - 1) / kMaxParts));
+  if (few)
+    r.l_min = vmin(r.l_cap, vmax(r.l_min, static_cast<int>(__builtin_sqrtf(0.5f * most_tiles) + 1.5f) & ~(kWaves - 1)));
   r.l_top = vmin(r.l_cap, vmax(r.l_min, most_tiles));
   r.l_fair = static_cast<int>(vmin<int64_t>(
       r.l_cap, vmax<int64_t>(r.l_min, div_nonneg(total_tiles * hkv + r.target - 1, r.target))));
