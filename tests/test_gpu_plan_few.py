@@ -2,8 +2,8 @@
 
 Fewer units than half the CUs: pieces of at least sqrt(tiles / 2) tiles of the
 longest sequence, to the nearest four, one group per CU up to 32 tiles per CU,
-else two. The bound both plan kernels pick must be the smallest one that fits under these
-rules (brute force), and the decode on it must match the oracle.
+else two. The bound both plan kernels pick must be the smallest one that fits
+under these rules (brute force), and the decode on it must match the oracle.
 """
 
 import math
