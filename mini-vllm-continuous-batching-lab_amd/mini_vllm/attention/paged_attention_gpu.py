@@ -1622,6 +1622,13 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
     hit = _cache_get("prefill", (block_table,), extra)
     if hit is not None:
         return hit
+    # a negative chunk would shift the rows of the sequences after it out of
+    # the tensors; a negative prefix hides the chunk's own first keys
+    for r, c, q in zip(rows, cached, qlens):
+        if q < 0 or (q > 0 and c < 0):
+            raise IndexError(f"prefill: block_table row {r} insufficient: invalid lengths "
+                             f"(cached {c}, chunk {q})")
+    cached = [max(c, 0) for c in cached]  # (below 0 only without a chunk: nothing is read)
     cus = _groups_per_cu(device, head_dim, dtype)[1]
     tokens = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cus,
                              lambda t: sum(-(-q // t) for q in qlens if q > 0) * num_kv_heads)
@@ -1655,6 +1662,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         if any(status.tolist()):
             _check_prefix_tables(host_bt.detach().to("cpu", torch.int64), rows, cached, block_size,
                                  num_blocks)
+            raise IndexError("block_table insufficient to cover the cached prefixes")
     ws = None
     if max_parts > 1:
         ws_bytes = lib.mv_paged_prefill_blocks_workspace_bytes(
@@ -1806,9 +1814,10 @@ def hip_prefill_attention(
     (causal, offset by the prefix), ``scale = head_dim ** -0.5``, query
     head h reads kv head ``h // n_rep``. Returns ``[sum(query_len), Hq, D]``
     in the query dtype. ``IndexError`` (message "insufficient") for a table
-    that cannot cover a prefix, as the reference's gather raises. q / k / v
-    may be column views of one fused QKV output. ``cached_len_before`` and
-    ``query_len`` are sequences of ints or int tensors.
+    that cannot cover a prefix, as the reference's gather raises, and for
+    negative lengths (a captured call reports both). q / k / v may be column
+    views of one fused QKV output. ``cached_len_before`` and ``query_len``
+    are sequences of ints or int tensors.
 
     While the current stream is being captured into a graph the lengths
     may stay on the device: the work list is then built by a device kernel
