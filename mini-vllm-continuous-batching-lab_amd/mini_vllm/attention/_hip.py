@@ -283,10 +283,8 @@ def _bind_native(lib: ctypes.CDLL, mvlaunch) -> None:
     try:
         from . import _mvtorch
     except ImportError:
-        native = None
         return
     if _mvtorch.ABI != ABI_VERSION:
-        native = None
         return
     _mvtorch.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in (
         lib.mv_paged_decode_write, lib.mv_paged_decode, lib.mv_kv_cache_write,
@@ -296,6 +294,8 @@ def _bind_native(lib: ctypes.CDLL, mvlaunch) -> None:
 
 def _bind_calls(lib: ctypes.CDLL) -> None:
     global decode_write, decode, cache_write, rope_write, plan, prefill, decode_write_step
+    global native, launcher
+    native = launcher = None
     ctypes_calls = (lib.mv_paged_decode_write, lib.mv_paged_decode, lib.mv_kv_cache_write,
                     lib.mv_rope_kv_cache_write, lib.mv_decode_plan)
     prefill = lib.mv_paged_prefill_blocks
@@ -317,10 +317,10 @@ def _bind_calls(lib: ctypes.CDLL) -> None:
     decode_write, decode, cache_write, rope_write, plan = (
         _mvlaunch.decode_write, _mvlaunch.decode, _mvlaunch.cache_write, _mvlaunch.rope_write,
         _mvlaunch.plan)
-    if hasattr(_mvlaunch, "prefill"):
+    if hasattr(_mvlaunch, "prefill"):  # (an older build of the module has none)
         _mvlaunch.bind_prefill(ctypes.cast(prefill, ctypes.c_void_p).value)
         prefill = _mvlaunch.prefill
-    _bind_native(lib, _mvlaunch)
+        _bind_native(lib, _mvlaunch)
     decode_write_step = (_mvlaunch.decode_write_step
                          if getattr(_mvlaunch, "STEP_WORDS", None) == STEP_WORDS else None)
 
@@ -341,7 +341,13 @@ def load(path: str | None = None) -> ctypes.CDLL:
             )
         lib = ctypes.CDLL(p)
         for name, (restype, argtypes) in SIGNATURES.items():
-            fn = getattr(lib, name)
+            try:
+                fn = getattr(lib, name)
+            except AttributeError:
+                raise RuntimeError(
+                    f"{p} has no {name}: an older build; rebuild it with "
+                    f"`python {os.path.join(_PKG_ROOT, 'build_lib.py')}`"
+                ) from None
             fn.restype = restype
             fn.argtypes = argtypes
         if lib.mv_abi_version() != ABI_VERSION:
