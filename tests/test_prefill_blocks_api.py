@@ -46,6 +46,20 @@ def test_wide_partials_are_published_before_the_counter(tmp_path):
         check_handoff(name, ins)
 
 
+@pytest.mark.skipif(_hipcc() is None, reason="hipcc not installed")
+def test_whole_fp32_stages_are_straight_line(tmp_path):
+    """fp32 at head_dim 64: Q K^T of a stage whose 8 sub-tiles are all seen
+    (16 MFMAs each) has no branch in it."""
+    ks = kernels(device_asm("paged_prefill.hip", tmp_path), "paged_prefill_kernelILi0ELi64E")
+    assert len(ks) == 2, sorted(ks)  # 2 table types
+    for name, ins in ks.items():
+        run = most = 0
+        for i in ins:
+            run = 0 if i.startswith(("s_cbranch", "s_branch")) else run + i.startswith("v_mfma")
+            most = max(most, run)
+        assert most >= 8 * 16, (name, most)
+
+
 def test_launcher_passes_every_argument_in_order():
     """The fast-call wrapper against a stand-in for mv_paged_prefill_blocks."""
     import ctypes
