@@ -995,22 +995,34 @@ struct PieceRules {
 // a wave 0.4 us (fp32: 0.85) per tile of its own piece, so the shortest pieces
 // that fill the slots are not the fastest. The bound is at least the root of
 // half the longest sequence's tiles, near where the two costs meet (half:
-// fp32's side of it), to the nearest whole round of the four waves: 5 tiles
-// take two rounds (fp32, 1 sequence of 1024: 6.6 us at 4 tiles, 7.6 at 5). Up
-// to kFewTilesPerCU tiles per CU one group per CU is enough: merges, not
-// streaming, are the bound there. us per call, before -> after (14 / 2 heads x
-// 64 bf16 unless noted): 4 sequences of 4096 15.1 -> 9.1, 8 of 2048 12.7 ->
-// 9.0, 2 of 8192 19.8 -> 9.5, 16 of 4096 (32 tiles per CU) 12.5 -> 10.6; 28 / 4
-// heads x 128, 2 of 4096 19.2 -> 11.3; fp32, 8 of 2048 14.3 -> 10.7; up to 1024
-// tokens the bound stays 4. Above 32 tiles per CU two groups per CU stream as
-// fast (16 of 8192: 16.5 either way), and from half the CUs' units on a unit
-// has few pieces anyway (32 of 2048, 28 / 4 x 128: 24.6 us either way).
+// fp32's side of it), in whole rounds of the four waves (down to a multiple of
+// 4, up where at most 1.5 tiles are missing): 5 tiles take two rounds (fp32, 1
+// sequence of 1024: 6.6 us at 4 tiles, 7.6 at 5). Up to kFewTilesPerCU tiles
+// per CU one group per CU is enough: merges, not streaming, are the bound
+// there. us per call, before -> after (14 / 2 heads x 64 bf16 unless noted): 4
+// sequences of 4096 15.1 -> 9.1, 8 of 2048 12.7 -> 9.0, 2 of 8192 19.8 -> 9.5,
+// 16 of 4096 (32 tiles per CU) 12.5 -> 10.6; 28 / 4 heads x 128, 2 of 4096 19.2
+// -> 11.3; fp32, 8 of 2048 14.3 -> 10.7; up to 1024 tokens the bound stays 4.
+// Above 32 tiles per CU two groups per CU stream as fast (16 of 8192: 16.5
+// either way), and from half the CUs' units on a unit has few pieces anyway (32
+// of 2048, 28 / 4 x 128: 24.6 us either way). Equal pieces of every unit, one
+// per CU, can leave CUs idle (96 units on 256 CUs: 2 pieces each, 192 CUs):
+// the busy ones then take at most kFewTilesPerBusyCU, else two groups per CU
+// are sooner (48 sequences of 1300, 41 tiles per busy CU: 11.0 us with one
+// group, 10.1 with two; of 1100, 34.5: 9.9 and 9.6; of 1000, 31.5: 9.0 and
+// 9.3; 24 of 2600, 240 CUs busy, 32.6: 10.5 and 11.3).
 constexpr int kFewTilesPerCU = 32;
+constexpr int kFewTilesPerBusyCU = 34;
 __device__ inline PieceRules piece_rules(int groups_per_cu, int cu_count, int bs_log2, int64_t units,
                                          int64_t total_tiles, int most_tiles, int hkv) {
   PieceRules r;
   const bool few = 2 * units < cu_count;
-  const int few_per_cu = few && total_tiles * hkv <= static_cast<int64_t>(kFewTilesPerCU) * cu_count ? 1 : kFewUnitsPerCU;
+  int few_per_cu = kFewUnitsPerCU;
+  if (few) {
+    const int u = vmax(1, static_cast<int>(units));
+    const int most = vmin(kFewTilesPerCU * cu_count, kFewTilesPerBusyCU * (cu_count / u * u));
+    if (total_tiles * hkv <= most) few_per_cu = 1;
+  }
   const int per_cu = units <= cu_count ? vmin(few_per_cu, vmax(1, groups_per_cu))
                                        : vmin(kManyUnitsPerCU, vmax(1, groups_per_cu));
   r.target = static_cast<int64_t>(per_cu) * vmax(1, cu_count);

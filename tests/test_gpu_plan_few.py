@@ -1,8 +1,9 @@
 """The plan's piece bound where few (sequence, kv head) units share the CUs.
 
 Fewer units than half the CUs: pieces of at least sqrt(tiles / 2) tiles of the
-longest sequence, to the nearest four, one group per CU up to 32 tiles per CU,
-else two. The bound both plan kernels pick must be the smallest one that fits
+longest sequence, down to a multiple of four (up where at most 1.5 are missing),
+one group per CU up to 32 tiles per CU and 34 per CU that equal pieces of every
+unit fill (192 of 256 for 96 units), else two. The bound both plan kernels pick must be the smallest one that fits
 under these rules (brute force), and the decode on it must match the oracle.
 """
 
@@ -22,7 +23,8 @@ def _bound(kv_lens, hkv, per_cu, cus):
     tiles = [(k + 15) // 16 for k in kv_lens]
     units, total, most = len(tiles) * hkv, sum(tiles), max(tiles)
     few = 2 * units < cus
-    target = cus * (1 if few and total * hkv <= 32 * cus else min(2, per_cu))
+    one = few and total * hkv <= min(32 * cus, 34 * (cus // units * units))
+    target = cus * (1 if one else min(2, per_cu))
     l_cap = 511
     l_min = min(l_cap, max(4, -(-most // 128), int(math.sqrt(most / 2) + 1.5) // 4 * 4 if few else 0))
     l_top = min(l_cap, max(l_min, most))
@@ -45,6 +47,8 @@ def _bound(kv_lens, hkv, per_cu, cus):
     (14, 2, 64, torch.bfloat16, [4096] * 16), (14, 2, 64, torch.bfloat16, [4112] * 16),
     (28, 4, 128, torch.bfloat16, [2048] * 8), (8, 8, 64, torch.float16, [300] * 15),
     (8, 8, 64, torch.float16, [300] * 16), (16, 1, 128, torch.float32, [30, 9000, 2]),
+    (14, 2, 64, torch.bfloat16, [1000] * 48), (14, 2, 64, torch.bfloat16, [1300] * 48),
+    (8, 8, 64, torch.float16, [1100] * 12), (12, 3, 64, torch.float16, [1300] * 32),
     (14, 2, 64, torch.bfloat16, [700] * 63), (14, 2, 64, torch.bfloat16, [700] * 64),
 ], ids=lambda v: str(v)[:24])
 def test_bound_and_decode(hq, hkv, d, dtype, lens):
