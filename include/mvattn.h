@@ -587,8 +587,9 @@ size_t mv_paged_prefill_blocks_workspace_bytes(int32_t num_units, int32_t max_pa
  * mv_paged_prefill_parts (max_parts > 1: items of 8 ints) with items of up to
  * tokens_per_item query tokens, 1 .. mv_prefill_block_tokens(.., wide). Items
  * of more than mv_prefill_block_tokens(.., 0) tokens run with 256 query rows
- * per work group: faster where the 128-row work groups would take more than
- * one round over the CUs. Same math and contract otherwise.
+ * per work group: half the copies of the keys, but half the work groups, so
+ * faster only where whole rounds over the CUs do not grow by it. Same math and
+ * contract otherwise.
  */
 int mv_paged_prefill_blocks(const void* query, int64_t q_stride_tok, int64_t q_stride_head,
                             const void* key, int64_t k_stride_tok, int64_t k_stride_head,

@@ -1,12 +1,13 @@
 // Prefill attention with 256 packed query rows per work group (the 16-bit
-// types; mv_prefill16.h): eight row waves and no key sets, for launches whose
-// 128-row work groups would not fit the CUs in one round. A pass over the keys
-// then serves twice the rows: half the copies into LDS and no set merge.
-// Measured against 128 rows (bf16 / fp16, units at 128 rows): 14 / 2 heads x
-// 64, 16 x (1536 + 512) (928 units) 82.5 -> 75.4 us; 28 / 4 x 128, 8 x (1000 +
-// 300) (544) 69.8 -> 64.0, one 8192-token prompt (1824) 473 -> 434. Where the
-// 128-row groups fit one round they win: 4 x (1536 + 512) at 14 / 2 x 64 (232
-// units) 26.6 against 53.6 us.
+// types; mv_prefill16.h): eight row waves and no key sets. A pass over the keys
+// serves twice the rows of a 128-row group: half the copies into LDS and no set
+// merge, but half the groups, each with its keys in one chain. Measured
+// against 128 rows (units of 128 rows; 256 CUs): where whole rounds over the
+// CUs come out alike it wins, 14 / 2 heads x 64 bf16, 16 x (1536 + 512) (928
+// units) 82.5 -> 75.4 us; 28 / 4 x 128, 7 x (1536 + 504) (784) 131 -> 108, one
+// 8192-token prompt (1824) 473 -> 434; where they do not it loses, 4 x (1536 +
+// 512) at 14 / 2 x 64 (232) 26.6 -> 53.6, 5120 tokens over 1536 at 8 / 8 x 64
+// fp16 (320) 68 -> 113, a 4608-token prompt at 14 / 2 x 64 (512) 56 -> 81.
 #include "mv_prefill16.h"
 
 namespace mv {

@@ -1537,6 +1537,16 @@ def prefill_key_parts(key_ends: Sequence[int], cu_count: int,
     return out
 
 
+def _prefill_blocks(cached: np.ndarray, qlens: np.ndarray, tokens: int):
+    """(sequence, first token, tokens, keys) of every block of ``tokens``
+    chunk tokens, each sequence's last block (the most keys) first."""
+    blocks = np.maximum(-(-qlens // tokens), 0)
+    seq = np.repeat(np.arange(len(qlens)), blocks)
+    t0 = (np.repeat(np.cumsum(blocks), blocks) - 1 - np.arange(len(seq))) * tokens
+    nt = np.minimum(tokens, qlens[seq] - t0)
+    return seq, t0, nt, cached[seq] + t0 + nt
+
+
 def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int, tpg: int,
                  cu_count: int, max_parts: int):
     """Sequence records and work list of a prefill launch.
@@ -1553,16 +1563,11 @@ def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int,
     if n:
         seqs[:, 1], seqs[:, 3] = cached, qlens
         seqs[1:, 2] = np.cumsum(qlens)[:-1]
-    blocks = np.maximum(-(-qlens // tpg), 0)
-    nu = int(blocks.sum()) * num_kv_heads
+    seq, t0, nt, unit_keys = _prefill_blocks(cached, qlens, tpg)
+    nu = len(seq) * num_kv_heads
     if nu == 0:
         return seqs, np.zeros((0, 4), dtype=np.int32), 0, 1
-    # (sequence, token block) from each sequence's last block (the most
-    # keys), every kv head of it in a row
-    seq = np.repeat(np.arange(n), blocks)
-    t0 = (np.repeat(np.cumsum(blocks), blocks) - 1 - np.arange(len(seq))) * tpg
-    nt = np.minimum(tpg, qlens[seq] - t0)
-    unit_keys = cached[seq] + t0 + nt
+    # every kv head of a (sequence, token block) in a row
     items = np.empty((len(seq), num_kv_heads, 4), dtype=np.int32)
     items[:, :, 0], items[:, :, 2], items[:, :, 3] = seq[:, None], t0[:, None], nt[:, None]
     items[:, :, 1] = np.arange(num_kv_heads)
@@ -1586,19 +1591,83 @@ def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int,
     return seqs, work, nu, most
 
 
-def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, units_of) -> int:
-    """Query tokens per work group of a prefill launch (``units_of(tokens)``
-    work groups, uncut): as many as 128 query rows hold while those work
-    groups fit the CUs in one round, else 256 (measured:
-    csrc/paged_prefill_wide.hip)."""
+# us of one prefill work group of the 16-bit types per head_dim, as (fixed,
+# per key): 128 query rows; 256 of which at most 128 are in use; 256. Fitted to
+# the ratio of the two widths' times over 353 launches of 257 to 1024 128-row
+# units (1 to 16 query heads per kv head, chunks of 1 to 20000 tokens, prefixes
+# of 0 to 3000): the width it picks is the faster one within 0.4 % in the mean
+# and 16 % at most, where always 256 loses 52 % at most and always 128 56 %.
+_PREFILL_GROUP_US = {64: ((4.5, .0100), (4.1, .0130), (4.1, .0180)),
+                     128: ((7.8, .0162), (6.4, .0180), (8.8, .0257))}
+PREFILL_WIDE_ROUNDS = 4  # rounds of 128-row work groups above which 256 rows are taken
+
+
+def _prefill_us(cost: np.ndarray, num_kv_heads: int, cu_count: int) -> float:
+    """Time of work groups of these costs, each ``num_kv_heads`` times, on
+    ``cu_count`` CUs, one on a CU at a time, the longest first: some CU takes
+    j + 1 of the first j CUs' worth and one more; and all are busy at best."""
+    c = np.sort(cost)[::-1]
+    first = c[np.arange(0, len(c) * num_kv_heads, cu_count) // num_kv_heads]
+    return max(float((first * np.arange(1, len(first) + 1)).max()),
+               float(c.sum()) * num_kv_heads / cu_count)
+
+
+def _prefill_block_tokens(num_q_heads, num_kv_heads, head_dim, dtype) -> Tuple[int, int]:
+    """Query tokens that 128 and 256 query rows of a work group hold (fp32:
+    one size)."""
     lib = _hip.load()
     shape = (num_q_heads, num_kv_heads, head_dim, _hip.MV_DTYPE[dtype])
-    tokens = lib.mv_prefill_block_tokens(*shape, 0)
-    if tokens == 0:
+    narrow = lib.mv_prefill_block_tokens(*shape, 0)
+    if narrow == 0:
         raise RuntimeError(
             f"prefill: {num_q_heads} query heads over {num_kv_heads} kv heads not supported"
         )
-    return tokens if units_of(tokens) <= cu_count else lib.mv_prefill_block_tokens(*shape, 1)
+    return narrow, lib.mv_prefill_block_tokens(*shape, 1)
+
+
+def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, cached, qlens) -> int:
+    """Query tokens per work group of a prefill launch: what 128 or 256 query
+    rows hold. 256 rows read the keys half as often, but halve the work groups
+    and run their keys in one chain instead of two: by the work groups' times
+    (``_PREFILL_GROUP_US``) over whole rounds on the CUs. us, 128 and 256 rows
+    (units of 128): a 5400-token prompt at 14 / 2 x 64 (600) 83 and 97; 14 x
+    (1536 + 504) (784) 80.2 and 71.4; 5120 tokens over 1536 at 8 / 8 x 64 (320)
+    68 and 113; 9 x 512 at 16 / 1 x 128 (576) 32.7 and 23.4. One round: 128
+    rows, whose two sets of waves share the keys, unless every chunk is one
+    block of few keys (28 / 4 x 128, 32 x (300 + 5): 12.1 and 10.9). Above
+    ``PREFILL_WIDE_ROUNDS`` rounds 256, which is faster but where most of its
+    rows are empty (9 % slower at 200 x (2000 + 40) at 14 / 2 x 64)."""
+    narrow, wide = _prefill_block_tokens(num_q_heads, num_kv_heads, head_dim, dtype)
+    if wide == narrow:
+        return narrow
+    (n0, n1), (l0, l1), (w0, w1) = _PREFILL_GROUP_US[head_dim]
+    units = sum(-(-q // narrow) for q in qlens if q > 0) * num_kv_heads
+    if units > PREFILL_WIDE_ROUNDS * cu_count:
+        return wide
+    if units <= cu_count:
+        if not 0 < max(qlens, default=0) <= narrow:
+            return narrow
+        keys = max(c + q for c, q in zip(cached, qlens) if q > 0)
+        return wide if l0 + l1 * keys < n0 + n1 * keys else narrow
+    cached, qlens = np.asarray(cached, dtype=np.int64), np.asarray(qlens, dtype=np.int64)
+    _, _, _, keys = _prefill_blocks(cached, qlens, narrow)
+    narrow_us = _prefill_us(n0 + n1 * keys, num_kv_heads, cu_count)
+    _, _, tokens, keys = _prefill_blocks(cached, qlens, wide)
+    cost = np.where(tokens <= narrow, l0 + l1 * keys, w0 + w1 * keys)
+    return wide if _prefill_us(cost, num_kv_heads, cu_count) < narrow_us else narrow
+
+
+def _prefill_tokens_fixed(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, rows, seqs) -> int:
+    """``_prefill_tokens`` of a launch whose lengths stay on the device: 256
+    rows above ``PREFILL_WIDE_ROUNDS`` rounds, and at head_dim 128 where the
+    chunks are one block each on average (there 256 rows lose at most 10 % over
+    long prefixes and gain up to 20 % over short ones; at 64 they lose up to
+    28 %)."""
+    narrow, wide = _prefill_block_tokens(num_q_heads, num_kv_heads, head_dim, dtype)
+    units = -(-rows // narrow) * num_kv_heads
+    if rows <= seqs * narrow:
+        return wide if head_dim == 128 else narrow
+    return wide if units > PREFILL_WIDE_ROUNDS * cu_count else narrow
 
 
 def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_q_heads,
@@ -1630,8 +1699,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
                              f"(cached {c}, chunk {q})")
     cached = [max(c, 0) for c in cached]  # (below 0 only without a chunk: nothing is read)
     cus = _groups_per_cu(device, head_dim, dtype)[1]
-    tokens = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cus,
-                             lambda t: sum(-(-q // t) for q in qlens if q > 0) * num_kv_heads)
+    tokens = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cus, cached, qlens)
     bt = block_table
     if bt.dim() != 2:
         bt = bt.reshape(-1, bt.shape[-1] if bt.dim() else 0)
@@ -1746,9 +1814,8 @@ def _prefill_device_plan(block_table, seq_indices, cached_len_before, query_len,
     hit = _cache_get("prefill_graph", tensors, extra)
     if hit is not None:
         return hit
-    tpg = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype,
-                          _groups_per_cu(device, head_dim, dtype)[1],
-                          lambda t: (-(-total_rows // t) + n) * num_kv_heads)
+    tpg = _prefill_tokens_fixed(num_q_heads, num_kv_heads, head_dim, dtype,
+                                _groups_per_cu(device, head_dim, dtype)[1], total_rows, n)
     bt = block_table
     if bt.dim() != 2:
         bt = bt.reshape(-1, bt.shape[-1] if bt.dim() else 0)

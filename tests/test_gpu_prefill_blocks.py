@@ -1,7 +1,7 @@
 """mv_paged_prefill_blocks' two work-group sizes against the oracle.
 
-The 16-bit prefill runs 128 packed query rows per work group, or 256 where the
-128-row work groups would not fit the CUs in one round. Sizes here are the
+The 16-bit prefill runs 128 or 256 packed query rows per work group, whichever
+its launch is faster with (test_prefill_width.py). Sizes here are the
 edges: chunks of one token, of a work group's tokens and one more or less;
 prefixes that end at, before and after a 16-key sub-tile, a 32-key tile and a
 stage (64 and 128 keys); wave rows that straddle the causal diagonal; query
@@ -93,14 +93,6 @@ def test_output_rows_not_16_byte_aligned(wide):
         torch.cuda.synchronize()
         outs.append(out[..., :d].clone())
     assert torch.equal(outs[0], outs[1])
-
-
-def test_size_rule(monkeypatch):
-    """256 rows exactly where the 128-row work groups exceed the CUs."""
-    args = (14, 2, 64, torch.bfloat16, 256)
-    assert pag._prefill_tokens(*args, lambda t: 256) == 18
-    assert pag._prefill_tokens(*args, lambda t: 257) == 36
-    assert pag._prefill_tokens(14, 2, 64, torch.float32, 256, lambda t: 10 ** 6) == 16
 
 
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32], ids=str)
