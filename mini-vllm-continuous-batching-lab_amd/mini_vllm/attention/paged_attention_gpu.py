@@ -1625,6 +1625,22 @@ def _prefill_block_tokens(num_q_heads, num_kv_heads, head_dim, dtype) -> Tuple[i
     return narrow, lib.mv_prefill_block_tokens(*shape, 1)
 
 
+def _prefill_short_tokens(n_rep: int, head_dim: int, narrow: int, cu_count: int,
+                          units_of) -> int:
+    """Query tokens per work group of a one-round launch over few keys: at
+    head_dim 128 what the fewest of 32, 64, 96 or 128 rows hold with which the
+    launch still takes one round (``units_of(tokens)`` work groups). The merge of
+    a group's two key sets costs 0.45 us there with 128 rows, in proportion to
+    them. us, 128 rows -> this: 28 / 4 heads, 37 tokens 8.4 -> 7.2, 4 x (50 + 64)
+    10.0 -> 8.7, 300 tokens 12.5 -> 11.6 (the kernel before the sets: 7.8, 9.3,
+    14.8)."""
+    if head_dim == 128:
+        for rows in (32, 64, 96):
+            if units_of(rows // n_rep) <= cu_count:
+                return rows // n_rep
+    return narrow
+
+
 def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, cached, qlens) -> int:
     """Query tokens per work group of a prefill launch: what 128 or 256 query
     rows hold. 256 rows read the keys half as often, but halve the work groups
@@ -1633,9 +1649,9 @@ def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, cached
     (units of 128): a 5400-token prompt at 14 / 2 x 64 (600) 83 and 97; 14 x
     (1536 + 504) (784) 80.2 and 71.4; 5120 tokens over 1536 at 8 / 8 x 64 (320)
     68 and 113; 9 x 512 at 16 / 1 x 128 (576) 32.7 and 23.4. One round: 128
-    rows, whose two sets of waves share the keys, unless every chunk is one
-    block of few keys (28 / 4 x 128, 32 x (300 + 5): 12.1 and 10.9). Above
-    ``PREFILL_WIDE_ROUNDS`` rounds 256, which is faster but where most of its
+    rows or fewer (``_prefill_short_tokens``), whose two sets of waves share the
+    keys, unless every chunk is one block of few keys (28 / 4 x 128, 32 x (300 +
+    5): 12.1 and 10.9). Above ``PREFILL_WIDE_ROUNDS`` rounds 256, which is faster but where most of its
     rows are empty (9 % slower at 200 x (2000 + 40) at 14 / 2 x 64)."""
     narrow, wide = _prefill_block_tokens(num_q_heads, num_kv_heads, head_dim, dtype)
     if wide == narrow:
@@ -1645,10 +1661,14 @@ def _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, cached
     if units > PREFILL_WIDE_ROUNDS * cu_count:
         return wide
     if units <= cu_count:
-        if not 0 < max(qlens, default=0) <= narrow:
+        keys = max((c + q for c, q in zip(cached, qlens) if q > 0), default=0)
+        if 0 < max(qlens, default=0) <= narrow and l0 + l1 * keys < n0 + n1 * keys:
+            return wide
+        if keys > 3 * PREFILL_PART_KEYS:  # (its keys may be cut into parts)
             return narrow
-        keys = max(c + q for c, q in zip(cached, qlens) if q > 0)
-        return wide if l0 + l1 * keys < n0 + n1 * keys else narrow
+        return _prefill_short_tokens(
+            num_q_heads // num_kv_heads, head_dim, narrow, cu_count,
+            lambda t: sum(-(-q // t) for q in qlens if q > 0) * num_kv_heads)
     cached, qlens = np.asarray(cached, dtype=np.int64), np.asarray(qlens, dtype=np.int64)
     _, _, _, keys = _prefill_blocks(cached, qlens, narrow)
     narrow_us = _prefill_us(n0 + n1 * keys, num_kv_heads, cu_count)
@@ -1667,7 +1687,10 @@ def _prefill_tokens_fixed(num_q_heads, num_kv_heads, head_dim, dtype, cu_count, 
     units = -(-rows // narrow) * num_kv_heads
     if rows <= seqs * narrow:
         return wide if head_dim == 128 else narrow
-    return wide if units > PREFILL_WIDE_ROUNDS * cu_count else narrow
+    if units > PREFILL_WIDE_ROUNDS * cu_count:
+        return wide
+    return _prefill_short_tokens(num_q_heads // num_kv_heads, head_dim, narrow, cu_count,
+                                 lambda t: (-(-rows // t) + seqs) * num_kv_heads)
 
 
 def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_q_heads,

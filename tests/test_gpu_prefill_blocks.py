@@ -65,6 +65,25 @@ def test_wide_key_parts_and_sharp_scores(monkeypatch, d):
         assert err <= TOL[torch.bfloat16], err
 
 
+@pytest.mark.parametrize("shape", [(14, 2, 64, torch.float16), (28, 4, 128, torch.bfloat16),
+                                   (16, 1, 128, torch.float16)], ids=str)
+@pytest.mark.parametrize("rows", [32, 64, 96, 128])
+def test_few_rows_and_few_keys(monkeypatch, shape, rows):
+    """Work groups of fewer rows (whose other waves have none), over key ranges
+    that end at, before and after the first 32 keys, the only ones the second
+    set of waves has no part in, and a stage."""
+    hq, hkv, d, dt = shape
+    say("prefill few rows", shape, rows)
+    cached = [0, 0, 0, 0, 31, 31, 32, 20, 64, 96, 127, 128]
+    qlen = [1, 31, 32, 33, 1, 2, 1, 9, 5, 33, 1, 2]
+    c = _case(hq, hkv, d, 16, dt, cached, qlen, seed=23)
+    monkeypatch.setattr(pag, "_prefill_tokens", lambda *a: rows * hkv // hq)
+    out = _run(c)
+    assert not torch.isnan(out).any()
+    err = (out - _ref(c)).abs().max().item()
+    assert err <= TOL[dt], err
+
+
 @pytest.mark.parametrize("wide", [0, 1])
 def test_output_rows_not_16_byte_aligned(wide):
     """The C ABI takes any output strides: element stores give the same bits

@@ -51,6 +51,21 @@ def test_one_round_keeps_128_rows():
         pag._prefill_tokens(17, 1, 64, torch.bfloat16, 256, [0], [5])
 
 
+def test_short_launches_take_the_fewest_rows_of_one_round():
+    """head_dim 128: 32, 64, 96 or 128 rows, as the CUs hold their groups; not
+    at 64, and not where keys are cut into parts."""
+    def tokens(heads, n, q, cached=0):
+        return pag._prefill_tokens(*heads, torch.bfloat16, 256, [cached] * n, [q] * n)
+
+    big = (28, 4, 128)  # 7 query heads per kv head: 4, 9, 13 and 18 tokens
+    assert tokens(big, 1, 37) == 4 and tokens(big, 1, 256) == 4   # 64 blocks x 4 heads
+    assert tokens(big, 1, 257) == 9 and tokens(big, 7, 75) == 9   # 7 x 9 x 4 = 252
+    assert tokens(big, 16, 42) == 13 and tokens(big, 21, 42) == 18
+    assert tokens((16, 1, 128), 1, 20) == 2 and tokens((6, 6, 128), 1, 200) == 32
+    assert tokens(big, 1, 37, 731) == 4 and tokens(big, 1, 37, 732) == 18  # 768 keys
+    assert tokens((14, 2, 64), 1, 37) == 18
+
+
 def test_width_of_a_launch_with_lengths_on_the_device():
     def fixed(rows, seqs, d):
         return pag._prefill_tokens_fixed(14, 2, d, torch.bfloat16, 256, rows, seqs)
@@ -59,7 +74,10 @@ def test_width_of_a_launch_with_lengths_on_the_device():
         assert fixed(18 * 512, 1, d) == 18  # 1024 units: four rounds
         assert fixed(18 * 512 + 1, 1, d) == 36
     assert fixed(18 * 40, 40, 64) == 18 and fixed(18 * 40, 40, 128) == 36
-    assert fixed(18 * 40 + 1, 40, 128) == 18
+    assert fixed(18 * 60 + 1, 60, 128) == 18
+    # one round of fewer rows: (blocks + sequences) x 2 heads
+    assert fixed(37, 1, 64) == 18 and fixed(37, 1, 128) == 4 and fixed(4 * 127, 1, 128) == 4
+    assert fixed(4 * 127 + 1, 1, 128) == 9
 
 
 def test_blocks_cover_every_token_once():
