@@ -29,6 +29,42 @@ def native():
     pg.invalidate_cached_metadata()
 
 
+class Counted:
+    """_mvtorch with the outcome of every launch noted: "launched", or "python"
+    where it left the call to the wrapper."""
+
+    LAUNCHES = ("decode_write", "decode", "cache_write", "rope_write", "prefill")
+
+    def __init__(self, module):
+        self.module, self.outcomes = module, []
+
+    def __getattr__(self, name):
+        fn = getattr(self.module, name)
+        if name not in self.LAUNCHES:
+            return fn
+
+        def call(*args):
+            out = fn(*args)
+            assert out is None or out is True or type(out) is not int, (name, out)
+            self.outcomes.append((name, "python" if out is None else "launched"))
+            return out
+
+        return call
+
+
+# What layers 2 and 3 of a step do, in order (the first makes the plan and the
+# checks). Strided: K, and Q unless RoPE made it anew, are left to the wrapper.
+OUTCOMES = {
+    ("calls", False): [("cache_write", "launched"), ("decode", "launched")],
+    ("calls", True): [("cache_write", "python"), ("decode", "python")],
+    ("rope_calls", False): [("rope_write", "launched"), ("decode", "launched")],
+    ("rope_calls", True): [("rope_write", "python"), ("decode", "launched")],
+    ("write", False): [("decode_write", "launched")], ("write", True): [("decode_write", "python")],
+    ("sublayer", False): [("decode_write", "launched")],
+    ("sublayer", True): [("decode_write", "python")],
+}
+
+
 def _step(form, dtype, strided):
     spec = WorkloadSpec("native", 14, 2, 64, 16, dtype, 5, ("fixed", [1, 17, 64, 300, 33]))
     d = to_device(make_case(spec, seed=31))
@@ -66,7 +102,10 @@ def _step(form, dtype, strided):
 @pytest.mark.parametrize("form", ["calls", "rope_calls", "write", "sublayer"])
 def test_same_bits_with_and_without(monkeypatch, form, dtype, strided):
     say("native launches", form, dtype, strided)
+    counted = Counted(_hip.native)
+    monkeypatch.setattr(_hip, "native", counted)
     on = _step(form, dtype, strided)
+    assert counted.outcomes == 2 * OUTCOMES[form, strided]
     pg.invalidate_cached_metadata()
     monkeypatch.setattr(_hip, "native", None)
     off = _step(form, dtype, strided)
@@ -135,10 +174,12 @@ def test_prefill_layers(monkeypatch):
     kc = torch.randn(8, 2, 16, 64, generator=g).to(torch.bfloat16).to(DEV)
     bt = torch.arange(8, device=DEV).view(2, 4)
     outs = []
-    for native in (_hip.native, None):
+    counted = Counted(_hip.native)
+    for native in (counted, None):
         monkeypatch.setattr(_hip, "native", native)
         pg.invalidate_cached_metadata()
         for x in (q, q, q.transpose(1, 2).contiguous().transpose(1, 2)):
             outs.append(pg.hip_prefill_attention(x, k, v, kc, kc, bt, [0, 1], [20, 0], [37, 23], 16))
     for x in outs[1:]:
         assert torch.equal(bits(x.cpu()), bits(outs[0].cpu()))
+    assert counted.outcomes == [("prefill", x) for x in ("launched", "launched", "python")]
