@@ -1514,29 +1514,6 @@ PREFILL_MAX_PARTS = 8     # key parts per prefill unit (mv_paged_prefill_parts)
 PREFILL_PART_KEYS = 256   # parts start at multiples of this many keys
 
 
-def prefill_key_parts(key_ends: Sequence[int], cu_count: int,
-                      max_parts: int = PREFILL_MAX_PARTS) -> List[List[Tuple[int, int]]]:
-    """Key ranges of the parts of each prefill unit (one (sequence, kv head,
-    token block) work group, whose rows see keys ``[0, key_end)``).
-
-    A launch of fewer units than ``cu_count`` leaves CUs idle, so each unit
-    is cut at multiples of ``PREFILL_PART_KEYS`` into up to
-    ``min(max_parts, cu_count // units)`` parts of at least two such blocks,
-    one work group each (``mv_paged_prefill_parts``). Returns
-    ``[(first key, end key), ...]`` per unit; ``[(0, key_end)]`` for a unit
-    that is not cut.
-    """
-    n = len(key_ends)
-    split = max(1, min(max_parts, cu_count // n)) if 0 < n < cu_count else 1
-    out = []
-    for ke in key_ends:
-        blocks = -(-ke // PREFILL_PART_KEYS)
-        parts = max(1, min(split, blocks // 2))
-        bounds = [(p * blocks // parts) * PREFILL_PART_KEYS for p in range(parts)] + [ke]
-        out.append([(bounds[p], bounds[p + 1]) for p in range(parts)])
-    return out
-
-
 def _prefill_blocks(cached: np.ndarray, qlens: np.ndarray, tokens: int):
     """(sequence, first token, tokens, keys) of every block of ``tokens``
     chunk tokens, each sequence's last block (the most keys) first."""
@@ -1551,10 +1528,14 @@ def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int,
                  cu_count: int, max_parts: int):
     """Sequence records and work list of a prefill launch.
 
-    Units are (sequence, kv head, block of ``tpg`` chunk tokens). Returns
-    ``(seqs, work, units, parts)``: int64 [n, 4] (0, cached, first chunk row,
-    chunk tokens), int32 [slots, 4 or 8] (8 when some unit is cut into parts,
-    ``prefill_key_parts``), the number of units and the most parts of one.
+    Units are (sequence, kv head, block of ``tpg`` chunk tokens), whose rows see
+    keys ``[0, key_end)``. A launch of fewer units than ``cu_count`` leaves CUs
+    idle, so each unit is cut at multiples of ``PREFILL_PART_KEYS`` into up to
+    ``min(max_parts, cu_count // units)`` parts of at least two such blocks, one
+    work group each (``mv_paged_prefill_parts``). Returns ``(seqs, work, units,
+    parts)``: int64 [n, 4] (0, cached, first chunk row, chunk tokens), int32
+    [slots, 4 or 8] (8 when some unit is cut), the number of units and the most
+    parts of one.
     """
     cached = np.asarray(cached, dtype=np.int64).reshape(-1)
     qlens = np.asarray(qlens, dtype=np.int64).reshape(-1)
@@ -1574,7 +1555,7 @@ def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int,
     items = items.reshape(nu, 4)
     keys = np.repeat(unit_keys, num_kv_heads)
     most = 1
-    if nu < cu_count:  # the parts of prefill_key_parts, unit by unit
+    if nu < cu_count:
         kb = -(-keys // PREFILL_PART_KEYS)
         count = np.clip(kb // 2, 1, max(1, min(max_parts, cu_count // nu)))
         most = int(count.max())
@@ -1703,7 +1684,7 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
     Work groups are (sequence, kv head, first token, tokens), the most keys
     first; per sequence (table row, cached, first chunk row, chunk tokens).
     When the units are fewer than the CUs their keys are cut into parts
-    (``prefill_key_parts``): the work groups then carry (first key, end key,
+    (``prefill_work``): the work groups then carry (first key, end key,
     unit, part | parts << 8 | max parts << 16) as well, and the plan its own
     workspace for the merge (counters zero). ``MVATTN_PREFILL_PARTS`` caps
     the parts per unit (1: no cut).

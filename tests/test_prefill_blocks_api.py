@@ -83,16 +83,23 @@ def test_launcher_passes_every_argument_in_order():
 
 
 def _work_by_loops(cached, qlens, hkv, tokens, cus, max_parts):
-    """The work list's definition, unit by unit."""
-    from mini_vllm.attention.paged_attention_gpu import prefill_key_parts
-
+    """The work list's definition, unit by unit: fewer units than CUs are cut at
+    multiples of 256 keys into as many parts as CUs per unit, of 512 keys or
+    more."""
     items, keys = [], []
     for i, (c, q) in enumerate(zip(cached, qlens)):
         for t0 in range(0, q, tokens):
             for h in range(hkv):
                 items.append((i, h, t0, min(tokens, q - t0)))
                 keys.append(c + t0 + items[-1][3])
-    return items, prefill_key_parts(keys, cus, max_parts)
+    split = max(1, min(max_parts, cus // len(keys))) if 0 < len(keys) < cus else 1
+    parts = []
+    for ke in keys:
+        blocks = -(-ke // 256)
+        n = max(1, min(split, blocks // 2))
+        bounds = [p * blocks // n * 256 for p in range(n)] + [ke]
+        parts.append(list(zip(bounds, bounds[1:])))
+    return items, parts
 
 
 @pytest.mark.parametrize("cached,qlens,hkv,tokens", [

@@ -1,10 +1,29 @@
-"""The prefill key split's plan (prefill_key_parts): which units are cut,
+"""The key split of a prefill work list (prefill_work): which units are cut,
 where, and into how many parts (host logic; the GPU tests check the
 results)."""
 import pytest
 
 from mini_vllm.attention.paged_attention_gpu import (PREFILL_MAX_PARTS, PREFILL_PART_KEYS,
-                                                     prefill_key_parts)
+                                                     prefill_work)
+
+
+def key_parts(key_ends, cus, max_parts=PREFILL_MAX_PARTS):
+    """Key ranges per unit, as the work list of one-token sequences that see
+    ``key_ends`` keys holds them."""
+    n = len(key_ends)
+    _, work, units, most = prefill_work([ke - 1 for ke in key_ends], [1] * n, 1, 1, cus, max_parts)
+    assert units == n
+    parts = [{} for _ in range(n)]
+    for item in work.tolist():
+        if len(item) == 4:
+            parts[item[0]][0] = (0, key_ends[item[0]])
+            continue
+        first, end, unit, word = item[4:]
+        assert unit == item[0] and word >> 16 == most
+        parts[unit][word & 0xff] = (first, end)
+    out = [[pr[p] for p in range(len(pr))] for pr in parts]
+    assert most == max((len(pr) for pr in out), default=1)
+    return out
 
 
 @pytest.mark.parametrize("key_ends,cus", [
@@ -16,7 +35,7 @@ from mini_vllm.attention.paged_attention_gpu import (PREFILL_MAX_PARTS, PREFILL_
     ([], 256),
 ])
 def test_parts_tile_each_unit(key_ends, cus):
-    parts = prefill_key_parts(key_ends, cus)
+    parts = key_parts(key_ends, cus)
     assert len(parts) == len(key_ends)
     n = len(key_ends)
     cap = min(PREFILL_MAX_PARTS, cus // n) if 0 < n < cus else 1
@@ -33,17 +52,17 @@ def test_parts_tile_each_unit(key_ends, cus):
 
 
 def test_split_only_when_units_leave_cus_idle():
-    assert [len(p) for p in prefill_key_parts([4096] * 256, 256)] == [1] * 256
-    assert [len(p) for p in prefill_key_parts([4096] * 128, 256)] == [2] * 128
-    assert [len(p) for p in prefill_key_parts([4096] * 64, 256)] == [4] * 64
-    assert [len(p) for p in prefill_key_parts([4096] * 2, 256)] == [PREFILL_MAX_PARTS] * 2
+    assert [len(p) for p in key_parts([4096] * 256, 256)] == [1] * 256
+    assert [len(p) for p in key_parts([4096] * 128, 256)] == [2] * 128
+    assert [len(p) for p in key_parts([4096] * 64, 256)] == [4] * 64
+    assert [len(p) for p in key_parts([4096] * 2, 256)] == [PREFILL_MAX_PARTS] * 2
     # short units stay whole: a part needs two blocks of keys
-    assert [len(p) for p in prefill_key_parts([511, 512, 1024], 256)] == [1, 1, 2]
-    assert prefill_key_parts([4096] * 64, 256, max_parts=1) == [[(0, 4096)]] * 64
+    assert [len(p) for p in key_parts([511, 512, 1024], 256)] == [1, 1, 2]
+    assert key_parts([4096] * 64, 256, max_parts=1) == [[(0, 4096)]] * 64
 
 
 def test_parts_are_balanced():
     for ke in (4096, 3600, 2049, 100000):
-        pr = prefill_key_parts([ke], 256)[0]
+        pr = key_parts([ke], 256)[0]
         sizes = [b - a for a, b in pr]
         assert max(sizes) - min(sizes) <= 2 * PREFILL_PART_KEYS
