@@ -605,6 +605,24 @@ int mv_paged_prefill_blocks(const void* query, int64_t q_stride_tok, int64_t q_s
                             size_t workspace_bytes, void* stream);
 
 /*
+ * The sequence records and the work list of a prefill launch, on the host (no
+ * device work; every pointer is host memory). A unit is a (sequence, kv head,
+ * block of tokens_per_item chunk tokens). A launch of fewer units than
+ * cu_count leaves CUs idle, so each unit's keys are then cut at multiples of
+ * 256 into up to min(max_parts, cu_count / units) parts of at least 512 keys.
+ * The items with the most keys come first.
+ *   rows, cached, query_len  int64[num_seqs], lengths not negative;
+ *   seqs        int64[4 * num_seqs], as mv_paged_prefill reads it;
+ *   work_items  capacity_ints ints (8 * max(units, cu_count) suffice): items of
+ *               8 ints if some unit is cut, else of 4;
+ *   info        int32[3]: items, units, the most parts of a unit (1: 4 ints).
+ */
+int mv_prefill_work_items(const int64_t* rows, const int64_t* cached, const int64_t* query_len,
+                          int32_t num_seqs, int32_t num_kv_heads, int32_t tokens_per_item,
+                          int32_t cu_count, int32_t max_parts, int64_t* seqs,
+                          int32_t* work_items, int64_t capacity_ints, int32_t* info);
+
+/*
  * The table check of a prefill plan: status[i] (int32[num_seqs], device) = 1
  * where sequence i of seqs (see mv_paged_prefill) has a table row outside
  * [0, bt_rows), a cached prefix that is negative or longer than max_blocks

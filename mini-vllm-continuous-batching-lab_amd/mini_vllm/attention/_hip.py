@@ -181,6 +181,11 @@ SIGNATURES = {
         _I32, _I32, _I32, _I64,    # bt_rows, max_blocks, block_size, num_blocks
         _P, _P,                    # status, stream
     ]),
+    "mv_prefill_work_items": (ctypes.c_int, [
+        _P, _P, _P, _I32, _I32,    # rows, cached, query_len, num_seqs, num_kv_heads
+        _I32, _I32, _I32,          # tokens_per_item, cu_count, max_parts
+        _P, _P, _I64, _P,          # seqs, work_items, capacity_ints, info
+    ]),
     "mv_prefill_block_tokens": (ctypes.c_int, [_I32, _I32, _I32, _I32, _I32]),
     "mv_paged_prefill_blocks_workspace_bytes": (ctypes.c_size_t, [_I32] * 7),
     "mv_paged_prefill_blocks": (ctypes.c_int, [

@@ -1512,6 +1512,10 @@ def _check_prefix_tables(bt_host: torch.Tensor, rows: Sequence[int], lens: Seque
 
 PREFILL_MAX_PARTS = 8     # key parts per prefill unit (mv_paged_prefill_parts)
 PREFILL_PART_KEYS = 256   # parts start at multiples of this many keys
+# A host table of up to this many sequences is checked on the host: a first
+# layer of 1 / 4 / 6 / 16 sequences takes 59 / 69 / 77 / 112 us then, 75 / 75 /
+# 75 / 80 with the check on the device and its read-back.
+PREFILL_HOST_CHECK_SEQS = 5
 
 
 def _prefill_blocks(cached: np.ndarray, qlens: np.ndarray, tokens: int):
@@ -1524,52 +1528,36 @@ def _prefill_blocks(cached: np.ndarray, qlens: np.ndarray, tokens: int):
     return seq, t0, nt, cached[seq] + t0 + nt
 
 
-def prefill_work(cached: Sequence[int], qlens: Sequence[int], num_kv_heads: int, tpg: int,
-                 cu_count: int, max_parts: int):
-    """Sequence records and work list of a prefill launch.
+def prefill_work(rows: Sequence[int], cached: Sequence[int], qlens: Sequence[int],
+                 num_kv_heads: int, tokens: int, cu_count: int, max_parts: int):
+    """Sequence records and work list of a prefill launch
+    (``mv_prefill_work_items``): ``(buffer, seqs, work, units, parts)`` with one
+    host int32 buffer, its int64 [n, 4] view of the records (table row, cached,
+    first chunk row, chunk tokens), its int32 [items, 4 or 8] view of the work
+    items (8 when some unit is cut into parts), the number of units and the most
+    parts of one."""
+    lib = _hip.load()
+    n = len(rows)
+    units = sum(-(-q // tokens) for q in qlens) * num_kv_heads
+    buf = torch.empty(8 * n + 8 * max(units, cu_count), dtype=torch.int32)
+    base = buf.data_ptr()
+    lists = (ctypes.c_int64 * (3 * n))(*rows, *cached, *qlens)
+    at = ctypes.addressof(lists)
+    info = (ctypes.c_int32 * 3)()
+    _hip.check(
+        lib.mv_prefill_work_items(at, at + 8 * n, at + 16 * n, n, num_kv_heads, tokens, cu_count,
+                                  max_parts, base, base + 32 * n, buf.numel() - 8 * n, info),
+        "mv_prefill_work_items",
+    )
+    items, units, most = info
+    ints = 8 if most > 1 else 4
+    buf = buf[:8 * n + ints * items]
+    return (buf, *_prefill_views(buf, n, ints), units, most)
 
-    Units are (sequence, kv head, block of ``tpg`` chunk tokens), whose rows see
-    keys ``[0, key_end)``. A launch of fewer units than ``cu_count`` leaves CUs
-    idle, so each unit is cut at multiples of ``PREFILL_PART_KEYS`` into up to
-    ``min(max_parts, cu_count // units)`` parts of at least two such blocks, one
-    work group each (``mv_paged_prefill_parts``). Returns ``(seqs, work, units,
-    parts)``: int64 [n, 4] (0, cached, first chunk row, chunk tokens), int32
-    [slots, 4 or 8] (8 when some unit is cut), the number of units and the most
-    parts of one.
-    """
-    cached = np.asarray(cached, dtype=np.int64).reshape(-1)
-    qlens = np.asarray(qlens, dtype=np.int64).reshape(-1)
-    n = len(qlens)
-    seqs = np.zeros((max(n, 1), 4), dtype=np.int64)
-    if n:
-        seqs[:, 1], seqs[:, 3] = cached, qlens
-        seqs[1:, 2] = np.cumsum(qlens)[:-1]
-    seq, t0, nt, unit_keys = _prefill_blocks(cached, qlens, tpg)
-    nu = len(seq) * num_kv_heads
-    if nu == 0:
-        return seqs, np.zeros((0, 4), dtype=np.int32), 0, 1
-    # every kv head of a (sequence, token block) in a row
-    items = np.empty((len(seq), num_kv_heads, 4), dtype=np.int32)
-    items[:, :, 0], items[:, :, 2], items[:, :, 3] = seq[:, None], t0[:, None], nt[:, None]
-    items[:, :, 1] = np.arange(num_kv_heads)
-    items = items.reshape(nu, 4)
-    keys = np.repeat(unit_keys, num_kv_heads)
-    most = 1
-    if nu < cu_count:
-        kb = -(-keys // PREFILL_PART_KEYS)
-        count = np.clip(kb // 2, 1, max(1, min(max_parts, cu_count // nu)))
-        most = int(count.max())
-    if most > 1:
-        unit = np.repeat(np.arange(nu), count)
-        part = np.arange(len(unit)) - np.repeat(np.cumsum(count) - count, count)
-        kb, cnt = kb[unit], count[unit]
-        first = part * kb // cnt * PREFILL_PART_KEYS
-        end = np.where(part + 1 == cnt, keys[unit], (part + 1) * kb // cnt * PREFILL_PART_KEYS)
-        split = np.stack([first, end, unit, part | cnt << 8 | most << 16], axis=1)
-        items = np.concatenate([items[unit], split.astype(np.int32)], axis=1)
-        keys = end - first
-    work = items[np.argsort(-keys, kind="stable")]  # the most keys first
-    return seqs, work, nu, most
+
+def _prefill_views(buf: torch.Tensor, n: int, ints: int):
+    """The records and the work items in ``prefill_work``'s buffer."""
+    return buf[:8 * n].view(torch.int64).view(n, 4), buf[8 * n:].view(-1, ints)
 
 
 # us of one prefill work group of the 16-bit types per head_dim, as (fixed,
@@ -1701,6 +1689,8 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         if q < 0 or (q > 0 and c < 0):
             raise IndexError(f"prefill: block_table row {r} insufficient: invalid lengths "
                              f"(cached {c}, chunk {q})")
+        if c >= 1 << 30:  # (no pool holds it; the launch counts keys in 32 bits)
+            raise IndexError(f"block_table row {r} insufficient to cover {c} tokens")
     cached = [max(c, 0) for c in cached]  # (below 0 only without a chunk: nothing is read)
     cus = _groups_per_cu(device, head_dim, dtype)[1]
     tokens = _prefill_tokens(num_q_heads, num_kv_heads, head_dim, dtype, cus, cached, qlens)
@@ -1713,12 +1703,14 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         bt = bt.to(torch.int64)
     if bt.numel() and bt.stride(1) != 1:
         bt = bt.contiguous()
-    seqs, work, units, max_parts = prefill_work(
-        cached, qlens, num_kv_heads, tokens, cus,
+    host, _, work, units, max_parts = prefill_work(
+        rows, cached, qlens, num_kv_heads, tokens, cus,
         int(os.environ.get("MVATTN_PREFILL_PARTS", PREFILL_MAX_PARTS)))
-    seqs[:, 0] = rows
-    meta = torch.from_numpy(seqs).to(device, non_blocking=True)
-    if any(cached):
+    meta, work = _prefill_views(host.to(device, non_blocking=True), len(rows), work.shape[1])
+    if (any(cached) and host_bt.device.type == "cpu"
+            and len(rows) <= PREFILL_HOST_CHECK_SEQS):
+        _check_prefix_tables(host_bt.detach().to(torch.int64), rows, cached, block_size, num_blocks)
+    elif any(cached):
         # every entry the prefixes need is a pool block: checked on the device,
         # what is wrong looked up on the host
         status = torch.empty(len(rows), dtype=torch.int32, device=device)
@@ -1742,13 +1734,11 @@ def _prefill_plan(block_table, rows, cached, qlens, block_size, num_blocks, num_
         # the plan's own merge workspace: its counters start at zero and every
         # launch leaves them so; the layers of a step share it on one stream
         ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=device)
-    plan = (bt, meta,
-            torch.from_numpy(work).to(device, non_blocking=True), len(work), tokens, units,
-            max_parts, ws)
+    plan = (bt, meta, work, work.shape[0], tokens, units, max_parts, ws)
     has_bt = bt.numel() > 0
     plan += (_hip.prefill_words(
         _ptr(bt) if has_bt else None, int(bt.dtype == torch.int64), bt.stride(0) if has_bt else 0,
-        _ptr(plan[1]), len(rows), _ptr(plan[2]), len(work), tokens, units, max_parts,
+        _ptr(meta), len(rows), _ptr(work), work.shape[0], tokens, units, max_parts,
         float(head_dim ** -0.5), num_q_heads, num_kv_heads, head_dim, block_size, num_blocks,
         _hip.MV_DTYPE[dtype], _ptr(ws), ws.numel() if ws is not None else 0, device.index),)
     _cache_put("prefill", (block_table,), extra, plan)

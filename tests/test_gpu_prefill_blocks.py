@@ -116,11 +116,12 @@ def test_output_rows_not_16_byte_aligned(wide):
 
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32], ids=str)
 @pytest.mark.parametrize("where", ["device", "host"])
-def test_prefix_entries_are_checked_on_the_device(dtype, where):
+def test_prefix_entries_are_checked_on_the_device(monkeypatch, dtype, where):
     """The plan's table check against its definition on the host: rows and
     prefixes outside the table, entries at the pool's edges, entries past the
     prefix that do not count; tables of either type, on either side."""
     say("prefill prefix check", dtype, where)
+    monkeypatch.setattr(pag, "PREFILL_HOST_CHECK_SEQS", 0)
     hq, hkv, d, bs, nb = 14, 2, 64, 16, 40
     good = torch.arange(2 * 6).view(2, 6)
     cases = [(good, [0, 1], [96, 5], True), (good, [1, 0], [0, 81], True),

@@ -109,10 +109,12 @@ def _work_by_loops(cached, qlens, hkv, tokens, cus, max_parts):
 def test_work_list_holds_every_unit_and_part_once(cached, qlens, hkv, tokens):
     from mini_vllm.attention.paged_attention_gpu import prefill_work
 
-    seqs, work, units, most = prefill_work(cached, qlens, hkv, tokens, 256, 8)
+    at = [5 * i + 3 for i in range(len(cached))]
+    buf, seqs, work, units, most = prefill_work(at, cached, qlens, hkv, tokens, 256, 8)
     items, parts = _work_by_loops(cached, qlens, hkv, tokens, 256, 8)
     starts = [sum(qlens[:i]) for i in range(len(qlens))]
-    assert seqs.tolist() == [[0, c, s, q] for c, s, q in zip(cached, starts, qlens)]
+    assert seqs.tolist() == [[r, c, s, q] for r, c, s, q in zip(at, cached, starts, qlens)]
+    assert seqs.data_ptr() == buf.data_ptr() and buf.numel() == 2 * seqs.numel() + work.numel()
     assert units == len(items)
     assert most == max((len(p) for p in parts), default=1)
     rows = work.tolist()
@@ -130,3 +132,33 @@ def test_work_list_holds_every_unit_and_part_once(cached, qlens, hkv, tokens):
             assert [ranges[p] for p in range(len(want))] == want
         size = [r[5] - r[4] for r in rows]
     assert size == sorted(size, reverse=True)  # the most keys first
+
+
+def test_work_list_errors_before_anything_is_written(lib):
+    """Sizes, null pointers, lengths and a capacity that the items exceed."""
+    import ctypes
+
+    def call(cached, qlens, hkv=2, tokens=18, cus=256, parts=8, cap=4096, null=()):
+        n = len(cached)
+        i64 = [(ctypes.c_int64 * max(n, 1))(*x) for x in ([0] * n, cached, qlens)]
+        seqs, work = (ctypes.c_int64 * (4 * n + 4))(), (ctypes.c_int32 * max(cap, 1))(*[7] * max(cap, 1))
+        info = (ctypes.c_int32 * 3)()
+        args = [*i64, n, hkv, tokens, cus, parts, seqs, work, cap, info]
+        for k in null:
+            args[k] = None
+        return lib.mv_prefill_work_items(*args), list(work), list(info)
+
+    bad = _hip.MV_ERR_INVALID_ARGUMENT
+    for kw in (dict(hkv=0), dict(tokens=0), dict(cus=0), dict(parts=256), dict(cap=-1)):
+        assert call([0], [5], **kw)[0] == bad, kw
+    for k in (0, 1, 2, 8, 9, 11):
+        assert call([0], [5], null=(k,))[0] == bad, k
+    for cached, qlens in (([-1], [5]), ([0, 0], [5, -1]), ([1 << 31], [5]), ([0], [1 << 31])):
+        rc, work, _ = call(cached, qlens)
+        assert rc == bad and set(work) == {7}
+    rc, work, _ = call([0], [18 * 300], cap=4 * 600 - 1)  # 600 units of 4 ints
+    assert rc == bad and set(work) == {7}
+    assert call([0], [18 * 300], cap=4 * 600)[2] == [600, 600, 1]
+    assert call([4000], [18], cap=8 * 256 - 1)[0] == bad  # 2 units, cut: up to 256 items of 8 ints
+    assert call([4000], [18], cap=8 * 256)[2] == [16, 2, 8]
+    assert call([], [])[2] == [0, 0, 1]

@@ -36,6 +36,12 @@ def test_negative_lengths_are_refused(cached, qlens):
         _plan(cached, qlens)
 
 
+@pytest.mark.parametrize("cached", [1 << 30, 1 << 31, 1 << 40])
+def test_prefixes_no_pool_holds_are_refused(cached):
+    with pytest.raises(IndexError, match="insufficient to cover"):
+        _plan([0, cached], [2, 2])
+
+
 def test_a_sequence_without_a_chunk_needs_no_prefix(monkeypatch):
     """Accepted as before: its prefix is never read."""
     for cached in ([0, 0], [-1, 0], [-40, 0]):
@@ -48,15 +54,31 @@ def test_a_flagged_prefix_never_reaches_the_launch(monkeypatch):
     the host finds nothing."""
 
     class Lib:
-        mv_prefill_block_tokens = staticmethod(pag._hip.load().mv_prefill_block_tokens)
+        def __getattr__(self, name):
+            return getattr(lib, name)
 
         @staticmethod
         def mv_prefill_prefix_check(*a):
             return 0
 
-    monkeypatch.setattr(pag._hip, "load", lambda: Lib)
+    lib, stub = pag._hip.load(), Lib()
+    monkeypatch.setattr(pag, "PREFILL_HOST_CHECK_SEQS", 0)
+    monkeypatch.setattr(pag._hip, "load", lambda: stub)
     monkeypatch.setattr(pag, "_stream", lambda device: 0)
     real = torch.empty
     monkeypatch.setattr(torch, "empty", lambda *a, **k: real(*a, **k).fill_(1))
     with pytest.raises(IndexError, match="insufficient"):
         _plan([16, 16], [2, 2])
+
+
+@pytest.mark.parametrize("seqs", [1, 2])
+def test_a_host_table_of_few_sequences_is_checked_on_the_host(monkeypatch, seqs):
+    monkeypatch.setattr(pag, "PREFILL_HOST_CHECK_SEQS", seqs)
+    assert _plan([64] * seqs, [2] * seqs)[3] > 0
+    for cached in (65, 4000):  # the rows hold 4 blocks of 16
+        with pytest.raises(IndexError, match="insufficient"):
+            _plan([16] * (seqs - 1) + [cached], [2] * seqs)
+    table = torch.tensor([[0, 1, 64, -1]] * seqs)  # 64 pool blocks
+    with pytest.raises(IndexError, match="not all pool blocks"):
+        pag._prefill_plan(table, list(range(seqs)), [33] * seqs, [1] * seqs, 16, 64, 14, 2, 64,
+                          torch.bfloat16, CPU)

@@ -11,7 +11,8 @@ def key_parts(key_ends, cus, max_parts=PREFILL_MAX_PARTS):
     """Key ranges per unit, as the work list of one-token sequences that see
     ``key_ends`` keys holds them."""
     n = len(key_ends)
-    _, work, units, most = prefill_work([ke - 1 for ke in key_ends], [1] * n, 1, 1, cus, max_parts)
+    _, _, work, units, most = prefill_work([0] * n, [ke - 1 for ke in key_ends], [1] * n, 1, 1, cus,
+                                           max_parts)
     assert units == n
     parts = [{} for _ in range(n)]
     for item in work.tolist():
