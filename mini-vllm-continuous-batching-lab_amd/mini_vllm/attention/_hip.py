@@ -270,16 +270,20 @@ def step_words(slots: int, rope_cos: int, rope_sin: int, work: int, ids: int, id
 # The words of _mvtorch.decode and _mvtorch.prefill: the step-constant
 # arguments of mv_paged_decode and mv_paged_prefill_blocks in their order, then
 # for prefill the device index.
-DECODE_WORDS_FORMAT = "<7qd9q"
-PREFILL_WORDS_FORMAT = "<10qd9q"
+_DECODE_WORDS = struct.Struct("<7qd9q")
+_PREFILL_WORDS = struct.Struct("<10qd9q")
 
 
 def decode_words(*args) -> bytes:
-    return struct.pack(DECODE_WORDS_FORMAT, *(a or 0 for a in args))
+    """mv_paged_decode's (the workspace, last but one, None if there is none)."""
+    return _DECODE_WORDS.pack(*args[:-2], args[-2] or 0, args[-1])
 
 
-def prefill_words(*args) -> bytes:
-    return struct.pack(PREFILL_WORDS_FORMAT, *(a or 0 for a in args))
+def prefill_words(block_table, *args) -> bytes:
+    """mv_paged_prefill_blocks' and the device index (the table, first, and the
+    workspace, last but two, None if there are none)."""
+    return _PREFILL_WORDS.pack(block_table or 0, *args[:-3], args[-3] or 0, args[-2],
+                               args[-1] or 0)
 
 
 def _bind_native(lib: ctypes.CDLL, mvlaunch) -> None:

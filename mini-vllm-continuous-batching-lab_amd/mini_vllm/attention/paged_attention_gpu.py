@@ -1174,28 +1174,25 @@ def hip_decode_attention(
             "mv_paged_decode_write",
         )
         return output
-    if not capture and _hip.native is not None:
-        # the other layers of the step launch from these words
-        plan.words[num_q_heads] = (
-            _hip.decode_words(
-                _ptr(plan.work), _ptr(plan.block_ids), plan.block_ids.numel(), plan.num_groups,
-                plan.partition_tokens, plan.max_parts, _ptr(plan.counters),
-                float(head_dim ** -0.5), total_decode, num_q_heads, num_kv_heads, head_dim,
-                block_size, num_blocks, _hip.MV_DTYPE[dtype], _ptr(ws),
-                ws.numel() if ws is not None else 0), ws)
+    split = (_ptr(plan.work), _ptr(plan.block_ids), plan.block_ids.numel(), plan.num_groups,
+             plan.partition_tokens, plan.max_parts, _ptr(plan.counters))
+    shape = (float(head_dim ** -0.5), total_decode, num_q_heads, num_kv_heads, head_dim,
+             block_size, num_blocks, _hip.MV_DTYPE[dtype])
+    space = (_ptr(ws), ws.numel()) if ws is not None else (None, 0)
     _hip.check(
         _hip.decode(
-            _ptr(query), query.stride(0), query.stride(1),
-            _ptr(key_cache), _ptr(value_cache),
-            _ptr(plan.work), _ptr(plan.block_ids), plan.block_ids.numel(), plan.num_groups,
-            plan.partition_tokens, plan.max_parts, _ptr(plan.counters),
-            _ptr(output), output.stride(0), output.stride(1),
-            float(head_dim ** -0.5), total_decode, num_q_heads, num_kv_heads, head_dim,
-            block_size, num_blocks, _hip.MV_DTYPE[dtype],
-            _ptr(ws), ws.numel() if ws is not None else 0, _stream(device),
+            _ptr(query), query.stride(0), query.stride(1), _ptr(key_cache), _ptr(value_cache),
+            *split, _ptr(output), output.stride(0), output.stride(1), *shape, *space,
+            _stream(device),
         ),
         "mv_paged_decode",
     )
+    if not capture and _hip.native is not None:
+        # the other layers of the step launch from these words (packed while
+        # this layer runs)
+        known = plan.words.get(num_q_heads)
+        if known is None or known[1] is not ws:
+            plan.words[num_q_heads] = (_hip.decode_words(*split, *shape, *space), ws)
     return output
 
 

@@ -151,6 +151,31 @@ def test_later_layers_are_refused_as_before(monkeypatch, form, change):
             call(**{k: f(args[k]) for k, f in change.items()})
 
 
+def test_launch_words_are_packed_once_per_step(monkeypatch):
+    """Also where every layer is left to the wrapper; and again when the merge
+    workspace that they point at was replaced by a larger one."""
+    say("native launches: words packed")
+    packed = []
+    real = _hip.decode_words
+    monkeypatch.setattr(_hip, "decode_words", lambda *a: packed.append(a) or real(*a))
+    spec = WorkloadSpec("native", 14, 2, 64, 16, torch.bfloat16, 2, ("fixed", [900, 1500]))
+    d = to_device(make_case(spec, seed=35))
+    q = d.query.transpose(1, 2).contiguous().transpose(1, 2)
+
+    def call():
+        return pg.hip_decode_attention(q, d.key_cache, d.value_cache, d.block_table, d.kv_len, 16)
+
+    first = call()
+    for _ in range(3):
+        assert torch.equal(bits(call().cpu()), bits(first.cpu()))
+    assert len(packed) == 1
+    ws = pg._workspace(DEV if DEV.index is not None else torch.device("cuda", 0), 1)
+    pg._workspace(ws.device, ws.numel() + 1)
+    for _ in range(2):
+        assert torch.equal(bits(call().cpu()), bits(first.cpu()))
+    assert len(packed) == 2 and packed[0][-2] != packed[1][-2]
+
+
 def test_changed_metadata_is_checked_again():
     """An in-place write to the step's slots, lengths or table is seen."""
     say("native launches: changed metadata")
