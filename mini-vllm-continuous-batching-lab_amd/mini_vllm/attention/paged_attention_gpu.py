@@ -17,7 +17,10 @@ distinct metadata tensor: the 24 layer calls of one engine step pass the
 same ``slot_mapping`` / ``kv_len_after`` / block-table tensor objects, so
 only the first call of a step synchronises. A tensor is recognised by
 object identity plus its in-place version counter, so an in-place update
-(``copy_``, ``fill_``, indexing assignment) triggers a fresh check.
+(``copy_``, ``fill_``, indexing assignment) triggers a fresh check. The
+exception is an eager prefill with its lengths on the device: its plan is
+looked up by the lengths' values, so every layer reads them back (both
+tensors in one copy).
 """
 
 from __future__ import annotations
@@ -2157,9 +2160,9 @@ class AttentionBackendGPU(AttentionBackend):
         rows: List[int] = [int(s) for g in groups for s in g.seq_indices]
         if not rows:
             return query
-        # Lengths stay tensors: read on the host per step (eager), or planned
-        # on the device inside a captured graph. One group's tensors are
-        # passed as they are, so the layers of a step share one plan.
+        # Lengths stay tensors: read back by every eager layer, which finds the
+        # step's plan by their values, or planned on the device inside a captured
+        # graph, where one group's tensors, passed as they are, share one plan.
         if len(groups) == 1:
             cached, qlens = groups[0].cached_len_before, groups[0].query_len
         else:

@@ -107,8 +107,8 @@ def test_prefill_matches_oracle(shape):
 
 def test_bench_step_shape():
     """The bench's own prefill step: 4 sequences x (1536 cached + 512 chunk)
-    at the Qwen2-0.5B shape in bf16 (256 whole work groups, every stage of
-    the lazy softmax reference), in a fused QKV buffer as the runner has it."""
+    at the Qwen2-0.5B shape in bf16 (232 work groups of up to 18 tokens, the
+    lazy softmax reference throughout), in a fused QKV buffer as the runner has it."""
     say("prefill: bench step 4 x (1536 + 512)")
     c = _case(14, 2, 64, 16, torch.bfloat16, [1536] * 4, [512] * 4, seed=9, fused=True)
     out = _run(c)
@@ -241,7 +241,7 @@ def test_key_split_is_deterministic_and_matches_whole_units(monkeypatch):
     assert (whole - _ref(c)).abs().max().item() <= TOL[torch.float32]
 
 
-# ---- the softmax reference: stages kept as computed, or redone exactly
+# ---- the softmax reference: tiles kept as computed, or computed again with it moved
 
 def _scaled(c, q_mul=1.0, k_mul=1.0, k_keys=None):
     """The case with Q (and K: all keys, or prefix positions k_keys of every
@@ -267,9 +267,9 @@ def _scaled(c, q_mul=1.0, k_mul=1.0, k_keys=None):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
 @pytest.mark.parametrize("d", [64, 128])
 def test_sharp_scores(dt, d):
-    """Q x 4: scores of a few tens in the exponent's units, so stage sums
-    leave [2^-12, 2^12] and those stages are computed exactly (reference
-    moved, O rescaled); head_dim 64 (two wave sets) and 128 (one)."""
+    """Q x 4: scores of a few tens in the exponent's units, so tiles' sums
+    exceed 2^12 and those tiles are computed again (reference moved, O
+    rescaled), in either of the two wave sets."""
     say("prefill sharp scores", dt, d)
     c = _scaled(_case(14, 2, d, 16, dt, [1536, 300, 0], [512, 40, 100], seed=11), q_mul=4.0)
     out = _run(c)
@@ -281,9 +281,9 @@ def test_sharp_scores(dt, d):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
 def test_late_key_with_a_far_higher_score(dt):
-    """16 prefix keys (positions 1200-1215) with K x 12: their stage's sums
+    """16 prefix keys (positions 1200-1215) with K x 12: their tile's sums
     overflow the range, the reference moves up by tens of units, and the
-    stages after it are kept as computed again (sums far below 1, l above)."""
+    tiles after it are kept as computed again (sums far below 1, l above)."""
     say("prefill late high key", dt)
     c = _scaled(_case(14, 2, 64, 16, dt, [1536, 1300], [512, 64], seed=12), k_mul=12.0,
                 k_keys=range(1200, 1216))
@@ -296,9 +296,8 @@ def test_late_key_with_a_far_higher_score(dt):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=str)
 def test_scores_far_below_zero(dt):
-    """Every score near -60 in the exponent's units: the first stage's sums
-    fall below 2^-12 and are computed exactly, which moves the reference
-    down to the row maximum."""
+    """Every score near -60 in the exponent's units: the first tile moves the
+    reference from its start, below every score, to the row maximum."""
     say("prefill negative scores", dt)
     c = _case(14, 2, 64, 16, dt, [700, 0], [300, 33], seed=13)
     c["q"] = (c["q"].abs() * 2 + 1).to(dt).float()
