@@ -84,6 +84,51 @@ def test_few_rows_and_few_keys(monkeypatch, shape, rows):
     assert err <= TOL[dt], err
 
 
+@pytest.mark.parametrize("heads,cached,qlen,later,tokens", [
+    ((28, 4, 128), [0], [37], [37], 4),                      # fewest rows of one round
+    ((28, 4, 128), [0, 40, 300], [5, 18, 2], [7, 9, 9], 36),  # one block each: 256 rows
+    ((28, 4, 128), [64] * 3, [100, 9, 50], [1, 150, 8], 4),
+    ((14, 2, 64), [0, 33], [80, 41], [121, 0], 18),
+], ids=str)
+def test_captured_widths(heads, cached, qlen, later, tokens):
+    """A captured launch, whose work list the device builds for the width fixed
+    by its rows and sequences: replays with the lengths of the capture and with
+    others of the same sum, eager work in between."""
+    hq, hkv, d = heads
+    say("prefill captured", heads, cached, qlen)
+    dt, n, t = torch.bfloat16, len(qlen), sum(qlen)
+    assert pag._prefill_tokens_fixed(*heads, dt, 256, t, n) == tokens
+    cases = [_case(hq, hkv, d, 16, dt, cached, ql, seed=24 + i) for i, ql in enumerate((qlen, later))]
+    c = cases[0]
+    dev = {k: c[k].to(dt).to(DEV) for k in ("q", "k", "v", "kc", "vc")}
+    bt = c["bt"].to(DEV)
+    cached_d, qlen_d = torch.tensor(cached, device=DEV), torch.tensor(qlen, device=DEV)
+
+    def run():
+        return pag.hip_prefill_attention(*(dev[k] for k in ("q", "k", "v", "kc", "vc")), bt,
+                                         c["rows"], cached_d, qlen_d, 16)
+
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    cid = pag.last_capture_id()
+    for i in (0, 1, 0, 1):
+        x = cases[i]
+        for k in ("q", "k", "v", "kc", "vc"):
+            dev[k].copy_(x[k].to(dt))
+        bt.copy_(x["bt"])
+        qlen_d.copy_(torch.tensor(x["qlen"]))
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        pag.check_deferred(cid)
+        err = (out[:sum(x["qlen"])].float().cpu() - _ref(x)).abs().max().item()
+        assert err <= TOL[dt], (i, err)
+    pag.clear_deferred(cid)
+
+
 @pytest.mark.parametrize("wide", [0, 1])
 def test_output_rows_not_16_byte_aligned(wide):
     """The C ABI takes any output strides: element stores give the same bits
